@@ -795,6 +795,16 @@ __device__ __forceinline__ void duo_dma4(uint32_t lds, const uint32_t (&v)[4], i
       : "s"(lds), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "s"(r), "s"(soff)
       : "memory", "scc");
 }
+// one of those loads: lane l writes lds + 16 l from voffset v + soff
+__device__ __forceinline__ void duo_dma1(uint32_t lds, uint32_t v, i32x4 r, uint32_t soff) {
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "s"(lds), "v"(v), "s"(r), "s"(soff)
+      : "memory");
+}
 // At most VM of this wave's vector-memory operations outstanding and its LDS
 // operations done, then s_barrier.
 template <int VM>
@@ -1002,6 +1012,182 @@ __global__ void __launch_bounds__(kDuoThreads, 2) fp8_gemm_duo_kernel(GemmParams
       }
       __builtin_amdgcn_raw_buffer_store_b128(u32x4{w[0], w[1], w[2], w[3]}, crs, (uint32_t)(r * p.ldc + n0 + cl0), 0, 0);
     }
+  }
+}
+
+// bf16 operands on the two-workgroup form: the same 128 x 256 tile, five-slot
+// ring, item protocol and two workgroups per CU as above, on rows of bf16 (a
+// k-step of 128 bytes is 64 elements).
+//
+// What bounds it: the matrix cores (per k-step and wave 1 M MAC against 24 KiB
+// of LDS reads, 0.4 of the LDS rate), so the MFMA is v_mfma_f32_32x32x16_bf16,
+// whose measured rate is 1.62 PFLOP/s against 1.23 for 16x16x32 (whole chip,
+// register operands).  Wave w owns all 128 rows and columns [64 w, 64 w + 64)
+// as 4 x 2 accumulators of 32 x 32 (128 registers); a lane reads chunk
+// 2 kk + lane / 32 of row lane % 32 for the step's MFMA kk, which is conflict
+// free under the same swizzle (16 lanes read 16 consecutive rows).  The W rows
+// are permuted in LDS so that a lane's 16 accumulators of one 32 x 32 block
+// are two runs of eight output columns: 16-byte stores.
+// Measured against the 128 x 128 tile kernel (event-timed, back to back):
+// 162 251 x 512 x 2048 (M, K, N) 542 -> 420 us, K = 1536, N = 512 with a
+// residual 389 -> 300, K = 2048, N = 512 421 -> 326 us (1.04 PFLOP/s); 37 429
+// rows 124 -> 102, 80 -> 70, 96 -> 83 us.  Below about 5 000 rows the tiles no
+// longer cover the chip and a tile's serial k-steps (0.87 us each; 0.70 on the
+// smaller tile) are the time: 1 027 rows, K = 2048: 23 -> 28 us.
+//
+// Column (within a 32-column block) of accumulator element e (0..15) of lane
+// half h; the MFMA's row index is i = 8 (e / 4) + 4 h + e % 4.
+__device__ __forceinline__ int duo32_col(int h, int e) { return 16 * (e >> 3) + 8 * h + (e & 7); }
+
+__device__ __forceinline__ f32x16 mfma32_bf16(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                 0, 0);
+}
+
+template <bool RESID>
+__global__ void __launch_bounds__(kDuoThreads, 2) bf16_gemm_duo_kernel(GemmParams p, int per_xcd) {
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[kDuoSlots][kDuoItem];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int xcd = (int)blockIdx.x & 7;
+  const int t = xcd * per_xcd + ((int)blockIdx.x >> 3);
+  if (t >= min((xcd + 1) * per_xcd, p.tiles_m * p.tiles_n)) return;
+  const int mt = t / p.tiles_n, nt = t - mt * p.tiles_n;
+  const int m0 = mt * kBM, n0 = nt * kWideBN, mrows = min(kBM, p.M - m0);
+  const int nk = p.K >> 7;  // K in bytes
+
+  uint32_t av[4], wv[2][4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int q = 64 * (4 * wave + j) + lane, r = q >> 3;
+    const uint32_t pos = (uint32_t)(((q & 7) ^ wide_swz(r)) * 16);
+    av[j] = (uint32_t)r * (uint32_t)p.lda + pos;
+    const int i = r & 31;  // MFMA row of this LDS row: accumulator 4 (i / 8) + i % 4 of half (i / 4) % 2
+    const int col = (r & ~31) + duo32_col((i >> 2) & 1, 4 * (i >> 3) + (i & 3));
+    wv[0][j] = (uint32_t)col * (uint32_t)p.ldw + pos;
+    wv[1][j] = (uint32_t)(128 + col) * (uint32_t)p.ldw + pos;
+  }
+  const i32x4 ars = rsrc_sgprs(p.A + (int64_t)m0 * p.lda, (uint32_t)((mrows - 1) * p.lda + p.K));
+  const i32x4 wrs = rsrc_sgprs(p.W + (int64_t)n0 * p.ldw, (uint32_t)((kWideBN - 1) * p.ldw + p.K));
+  const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)&ring[0][0];
+  const int nitems = 3 * nk;
+  auto issue = [&](int it) {  // item it: k-step it / 3; 0 A, 1 W0, 2 W1
+    const int s = it / 3, kind = it - 3 * s;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(ring0 + (uint32_t)((it % kDuoSlots) * kDuoItem + 4096 * wave));
+    if (kind == 0) duo_dma4(dst, av, ars, (uint32_t)(s * 128));
+    else duo_dma4(dst, wv[kind - 1], wrs, (uint32_t)(s * 128));
+  };
+  for (int it = 0; it < min(5, nitems); ++it) issue(it);
+
+  const int lr = lane & 31, h = lane >> 5;
+  // chunk 2 kk + h of row lr of an even 32-row block; in odd blocks the
+  // swizzle flips bit 2, i.e. kk and kk ^ 2 trade places
+  uint32_t rd[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) rd[kk] = lr * 128 + (((2 * kk + h) ^ wide_swz(lr)) * 16);
+  const uint32_t w_off = 64 * (wave & 1) * 128;
+
+  // the lane's bias runs: columns 64 wave + 32 nb + 16 run + 8 h + (0..7)
+  const int cl = n0 + 64 * wave + 8 * h;
+  u32x4 bv[2][2];
+  auto load_consts = [&]() {
+    const BufRsrc bsr = make_rsrc(p.bias, p.bias ? (uint32_t)p.N * 2u : 0u);  // no bias: zeros
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int run = 0; run < 2; ++run) bv[nb][run] = buf_ld128(bsr, (uint32_t)(cl + 32 * nb + 16 * run) * 2u, 0);
+  };
+
+  f32x16 acc[4][2];
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.f;
+  auto read_block = [&](const uint8_t* st, int blk, u32x4 (&x)[4]) {
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) x[kk] = lds_ld128(st + 4096 * blk + rd[blk & 1 ? kk ^ 2 : kk]);
+  };
+  // one k-step; ITEMS: how many items are left to issue (3; 1 at step nk - 2;
+  // 0 at the last, which loads the epilogue constants instead).  All operands
+  // go to registers first, which frees the step's slots before its MFMAs; the
+  // DMAs are spread one per two MFMAs, because a wave that issues its twelve
+  // in a row waits at the texture address unit for the other waves' (48 KiB
+  // of loads) before its next MFMA.
+  auto kstep = [&](int s, auto items_c) {
+    constexpr int ITEMS = decltype(items_c)::value;
+    if constexpr (ITEMS == 0) duo_barrier<0>();
+    else duo_barrier<8>();
+    const uint8_t* sa_ = ring[(3 * s) % kDuoSlots];
+    const uint8_t* sw_ = ring[(3 * s + 1 + (wave >> 1)) % kDuoSlots] + w_off;
+    u32x4 w[2][4], a[4][4];
+    read_block(sw_, 0, w[0]);
+    read_block(sw_, 1, w[1]);
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) read_block(sa_, mb, a[mb]);
+    pc_barrier_lds();  // every wave has read step s: its three slots are free
+    if constexpr (ITEMS == 0) load_consts();
+    const uint32_t ka = (uint32_t)(128 * (s + 2)), kw1 = (uint32_t)(128 * (s + 1));
+    uint32_t dst[3];
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k)
+      dst[k] = __builtin_amdgcn_readfirstlane(ring0 + (uint32_t)(((3 * s + 5 + k) % kDuoSlots) * kDuoItem + 4096 * wave));
+    static_for<32>([&](auto nc) {
+      constexpr int n = decltype(nc)::value, mb = n >> 3, kk = (n >> 1) & 3, nb = n & 1;
+      acc[mb][nb] = mfma32_bf16(w[nb][kk], a[mb][kk], acc[mb][nb]);
+      if constexpr ((n & 1) == 1 && (n >> 1) < 4 * ITEMS) {  // items 3 s + 5 (W1), 3 s + 6 (A), 3 s + 7 (W0)
+        constexpr int k = n >> 3, j = (n >> 1) & 3;
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (k == 0) duo_dma1(dst[0] + 1024 * j, wv[1][j], wrs, kw1);
+        else if constexpr (k == 1) duo_dma1(dst[1] + 1024 * j, av[j], ars, ka);
+        else duo_dma1(dst[2] + 1024 * j, wv[0][j], wrs, ka);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+  };
+  for (int s = 0; s < nk - 2; ++s) kstep(s, std::integral_constant<int, 3>{});
+  kstep(nk - 2, std::integral_constant<int, 1>{});
+  kstep(nk - 1, std::integral_constant<int, 0>{});
+
+  // epilogue: lane holds C[m0 + 32 mb + lr][cl + 32 nb + 16 run + (0..7)];
+  // rows past M are dropped (stores) or read as zero (residual) by the range
+  // check of the buffer resources
+  const BufRsrc crs = make_rsrc((uint8_t*)p.C + (int64_t)m0 * p.ldc * 2, (uint32_t)(mrows * p.ldc * 2));
+  const BufRsrc rrs = make_rsrc(RESID ? (const void*)(p.resid + (int64_t)m0 * p.ldr) : p.C,
+                                RESID ? (uint32_t)(mrows * p.ldr * 2) : 0u);
+  const int wc0 = n0 + 64 * wave;
+  const bool silu = wc0 >= p.silu_begin && wc0 < p.silu_end;
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb) {
+    const int r = 32 * mb + lr;
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int run = 0; run < 2; ++run) {
+        const int c = cl + 32 * nb + 16 * run;
+        float o[8];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t b = bv[nb][run][j];
+          o[2 * j] = acc[mb][nb][8 * run + 2 * j] + bf16_to_f32((uint16_t)(b & 0xffff));
+          o[2 * j + 1] = acc[mb][nb][8 * run + 2 * j + 1] + bf16_to_f32((uint16_t)(b >> 16));
+        }
+        if (silu) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) o[e] = o[e] * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-kLog2e * o[e]));
+        }
+        if constexpr (RESID) {
+          const u32x4 rv = buf_ld128(rrs, (uint32_t)(r * p.ldr + c) * 2, 0);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            o[2 * j] += bf16_to_f32(rv[j] & 0xffff);
+            o[2 * j + 1] += bf16_to_f32(rv[j] >> 16);
+          }
+        }
+        __builtin_amdgcn_raw_buffer_store_b128(
+            u32x4{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3]), pack_bf16(o[4], o[5]), pack_bf16(o[6], o[7])}, crs,
+            (uint32_t)(r * p.ldc + c) * 2, 0, 0);
+      }
   }
 }
 
@@ -1586,6 +1772,21 @@ extern "C" int hstu_bf16_gemm(const void* A, int64_t lda, const void* W, int64_t
   p.silu_begin = silu_begin;
   p.silu_end = silu_end;
   p.tiles_m = (M + kBM - 1) / kBM;
+  // two-workgroup form: whole 256-column tiles, at least two k-steps, 16-byte
+  // output and residual rows, a SiLU range of whole waves (64 columns).  The
+  // rule does not look at M, so a row's bytes do not depend on its batch.
+  const bool duo_ok = N % kWideBN == 0 && p.K >= 2 * kBK && (uintptr_t)C % 16 == 0 && ldc % 8 == 0 &&
+                      (!residual || ((uintptr_t)residual % 16 == 0 && ldr % 8 == 0)) &&
+                      (silu_begin >= silu_end || (silu_begin % 64 == 0 && silu_end % 64 == 0)) &&
+                      (int64_t)kBM * 2 * ldc <= 0xffffffffLL && (int64_t)kBM * 2 * ldr <= 0xffffffffLL &&
+                      (int64_t)(kWideBN - 1) * p.ldw + p.K <= 0xffffffffLL;
+  if (duo_ok) {
+    p.tiles_n = N / kWideBN;
+    int per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
+    void* args[] = {&p, &per_xcd};
+    const void* dk = residual ? (const void*)bf16_gemm_duo_kernel<true> : (const void*)bf16_gemm_duo_kernel<false>;
+    return (int)hipLaunchKernel(dk, dim3(8 * per_xcd), dim3(kDuoThreads), args, 0, stream);
+  }
   p.tiles_n = N / kBN;
   void (*kern)(GemmParams) = residual ? fp8_gemm_kernel<false, true, kBF16> : fp8_gemm_kernel<false, false, kBF16>;
   hipError_t e = set_gemm_lds((const void*)kern);

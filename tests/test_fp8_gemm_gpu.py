@@ -310,3 +310,31 @@ def test_bf16_gemm_rows_independent_of_batch(hip_lib):
     part = fp8.bf16_gemm(a[1000:1300], w)
     torch.cuda.synchronize()
     assert torch.equal(full[1000:1300], part)
+
+
+@pytest.mark.parametrize("M,N,K,resid,pad", [(1, 256, 128, True, 0), (127, 512, 192, False, 0), (129, 256, 320, True, 8),
+                                             (385, 768, 128, False, 8), (200, 256, 64, False, 0),
+                                             (200, 256, 128, True, 4)])
+def test_bf16_gemm_two_workgroup_form(hip_lib, M, N, K, resid, pad):
+    """The two-workgroup bf16 form at its edges: two and three k-steps, ragged
+    last row tiles, strided rows; one k-step and 8-byte aligned output rows
+    (``pad`` 4) take the tile kernel.  Against the float64 product: relative
+    L2 <= 4e-3 (one bf16 rounding of a fp32 sum is 1.7e-3), SiLU on the second
+    64 columns, columns outside the output untouched."""
+    fp8 = _fp8()
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(M, K + 16, generator=g).to(torch.bfloat16)[:, 8:K + 8]
+    w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16)
+    b = (0.1 * torch.randn(N, generator=g)).to(torch.bfloat16)
+    r = torch.randn(M, N, generator=g).to(torch.bfloat16) if resid else None
+    wide = torch.full((M, N + pad + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    ad = torch.empty(M, K + 16, dtype=torch.bfloat16, device=DEV)[:, 8:K + 8]
+    ad.copy_(a)
+    fp8.bf16_gemm(ad, w.to(DEV), bias=b.to(DEV), residual=None if r is None else r.to(DEV), silu_cols=(64, 128),
+                  out=wide[:, :N])
+    ref = a.double() @ w.double().t() + b.double()
+    ref[:, 64:128] = torch.nn.functional.silu(ref[:, 64:128])
+    if r is not None:
+        ref = ref + r.double()
+    assert orc.rel_l2(ref, wide[:, :N].cpu().double()) <= 4e-3
+    assert bool((wide[:, N:] == 7.0).all())
