@@ -1031,9 +1031,9 @@ __global__ void __launch_bounds__(kDuoThreads, 2) fp8_gemm_duo_kernel(GemmParams
 // Measured against the 128 x 128 tile kernel (event-timed, back to back):
 // 162 251 x 512 x 2048 (M, K, N) 542 -> 420 us, K = 1536, N = 512 with a
 // residual 389 -> 300, K = 2048, N = 512 421 -> 326 us (1.04 PFLOP/s); 37 429
-// rows 124 -> 102, 80 -> 70, 96 -> 83 us.  Below about 5 000 rows the tiles no
-// longer cover the chip and a tile's serial k-steps (0.87 us each; 0.70 on the
-// smaller tile) are the time: 1 027 rows, K = 2048: 23 -> 28 us.
+// rows 124 -> 102, 80 -> 70, 96 -> 83 us.  With few rows the tiles no longer
+// cover the chip and a tile's serial k-steps (0.87 us each) are the time; those
+// calls take gemm_few_rows_kernel.
 //
 // Column (within a 32-column block) of accumulator element e (0..15) of lane
 // half h; the MFMA's row index is i = 8 (e / 4) + 4 h + e % 4.
@@ -1188,6 +1188,194 @@ __global__ void __launch_bounds__(kDuoThreads, 2) bf16_gemm_duo_kernel(GemmParam
             u32x4{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3]), pack_bf16(o[4], o[5]), pack_bf16(o[6], o[7])}, crs,
             (uint32_t)(r * p.ldc + c) * 2, 0, 0);
       }
+  }
+}
+
+// ---------------------------------------------------------------- few-row form
+// With few rows the 128 x 256 tiles leave most CUs idle and the time is one
+// tile's serial k-steps.  This form takes 64 x 64 tiles (4 waves of 32 x 32,
+// two workgroups per CU), eight times as many, and a ring of four 16 KiB stages
+// (A and W: 64 rows x 128 bytes each), so three k-steps' loads are in flight
+// and a step costs its LDS reads and MFMAs, not a memory round trip.  One
+// barrier per step: it publishes step s and frees step s - 1's stage, which
+// the loads of step s + 3 then take.  Every element is the same chain of the
+// same MFMAs over k as in the other forms (fp8: 16x16x128; bf16: 32x32x16 as
+// in bf16_gemm_duo_kernel), so the bytes are the same.
+// W rows are permuted in LDS so that a lane's accumulators of one row are
+// runs of eight output columns.
+// Measured (us, wide form before): 1 027 rows, e4m3 K = 1536, N = 512 with a
+// residual 16.7 -> 5.5, K = 512, N = 2048 8.6 -> 5.8; bf16 K = 2048, N = 512
+// 27.6 (the 128 x 128 tile kernel 23.2) -> 10.7; 33 rows, e4m3 K = 512,
+// N = 1536 7.1 -> 3.0.
+constexpr int kFewB = 64, kFewStages = 4, kFewStage = 2 * kFewB * 128;
+
+template <bool E4M3_OUT, bool RESID, int FMT>
+__global__ void __launch_bounds__(kThreads, 2) gemm_few_rows_kernel(GemmParams p) {
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[kFewStages][kFewStage];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  // XCD x runs a contiguous range of tiles, column-panel-major: an XCD's L2
+  // then holds its share of W and all of A (few rows: W is the larger)
+  const int total = p.tiles_m * p.tiles_n, per_xcd = (total + 7) / 8;
+  const int t = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
+  if (t >= min((((int)blockIdx.x & 7) + 1) * per_xcd, total)) return;
+  const int nt = t / p.tiles_m, mt = t - nt * p.tiles_m;
+  const int m0 = mt * kFewB, n0 = nt * kFewB, mrows = min(kFewB, p.M - m0);
+  const int wm = 32 * (wave >> 1), wn = 32 * (wave & 1);
+  const int nk = p.K >> 7;  // K in bytes
+  const int li = lane & 15, g = lane >> 4, lr = lane & 31, h = lane >> 5;
+  // run `run` of the lane's accumulators starts at this column of the wave's
+  // 32; fp8: one run per row block ms, bf16: two runs of one row
+  const int c0 = n0 + wn + (FMT == kBF16 ? 8 * h : 8 * g);
+
+  // epilogue constants, loaded first: they land under the k-loop
+  f32x4 sw[2];
+  u32x4 bv[2];
+  float sa[2];
+  {
+    const BufRsrc bsr = make_rsrc(p.bias, p.bias ? (uint32_t)p.N * 2u : 0u);  // no bias: zeros
+    bv[0] = buf_ld128(bsr, (uint32_t)c0 * 2u, 0);
+    if constexpr (FMT == kBF16) {
+      bv[1] = buf_ld128(bsr, (uint32_t)(c0 + 16) * 2u, 0);
+    } else {
+      if (p.w_mode) {
+        const BufRsrc swr = make_rsrc(p.w_scale, (uint32_t)p.N * 4u);
+        sw[0] = __builtin_bit_cast(f32x4, buf_ld128(swr, (uint32_t)c0 * 4u, 0));
+        sw[1] = __builtin_bit_cast(f32x4, buf_ld128(swr, (uint32_t)c0 * 4u + 16u, 0));
+      } else {
+        const float s0 = p.w_scale[0];
+        sw[0] = sw[1] = f32x4{s0, s0, s0, s0};
+      }
+#pragma unroll
+      for (int ms = 0; ms < 2; ++ms) sa[ms] = p.a_mode ? p.a_scale[min(m0 + wm + 16 * ms + li, p.M - 1)] : p.a_scale[0];
+    }
+  }
+
+  // DMA sources: wave w fills rows 16 w .. 16 w + 15 of both operands' stages
+  uint32_t av[2], wv[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int q = 64 * (2 * wave + j) + lane, r = q >> 3, b = r & ~31;
+    const uint32_t pos = (uint32_t)(((q & 7) ^ wide_swz(r)) * 16);
+    int col;
+    if constexpr (FMT == kBF16) {
+      const int i = r & 31;
+      col = b + duo32_col((i >> 2) & 1, 4 * (i >> 3) + (i & 3));
+    } else {
+      const int i = r & 15;  // row block ns = (r >> 4) & 1: accumulators 4 ns + i % 4 of group i / 4
+      col = b + 8 * (i >> 2) + 4 * ((r >> 4) & 1) + (i & 3);
+    }
+    av[j] = (uint32_t)r * (uint32_t)p.lda + pos;
+    wv[j] = (uint32_t)col * (uint32_t)p.ldw + pos;
+  }
+  const i32x4 ars = rsrc_sgprs(p.A + (int64_t)m0 * p.lda, (uint32_t)((mrows - 1) * p.lda + p.K));
+  const i32x4 wrs = rsrc_sgprs(p.W + (int64_t)n0 * p.ldw, (uint32_t)((kFewB - 1) * p.ldw + p.K));
+  const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)&ring[0][0];
+  auto issue = [&](int s) {  // four loads of this wave: A, A, W, W
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(ring0 + (uint32_t)((s % kFewStages) * kFewStage + 2048 * wave));
+#pragma unroll
+    for (int j = 0; j < 2; ++j) duo_dma1(dst + 1024 * j, av[j], ars, (uint32_t)(128 * s));
+#pragma unroll
+    for (int j = 0; j < 2; ++j) duo_dma1(dst + kFewStage / 2 + 1024 * j, wv[j], wrs, (uint32_t)(128 * s));
+  };
+  for (int s = 0; s < min(kFewStages - 1, nk); ++s) issue(s);
+
+  f32x4 acc4[2][2];
+  f32x16 acc16;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc4[i >> 1][i & 1] = zero4();
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc16[r] = 0.f;
+  auto kstep = [&](int s, auto vm_c) {
+    // step s has landed when only the loads of the (up to two) later steps
+    // issued so far are outstanding
+    duo_barrier<decltype(vm_c)::value>();
+    if (s + kFewStages - 1 < nk) issue(s + kFewStages - 1);
+    const uint8_t* sa_ = ring[s % kFewStages] + wm * 128;
+    const uint8_t* sw_ = ring[s % kFewStages] + kFewStage / 2 + wn * 128;
+    if constexpr (FMT == kBF16) {
+      u32x4 a[4], w[4];
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        a[kk] = lds_ld128(sa_ + lr * 128 + (((2 * kk + h) ^ wide_swz(wm + lr)) * 16));
+        w[kk] = lds_ld128(sw_ + lr * 128 + (((2 * kk + h) ^ wide_swz(wn + lr)) * 16));
+      }
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) acc16 = mfma32_bf16(w[kk], a[kk], acc16);
+    } else {
+      i32x8 a[2], w[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int r = 16 * i + li;
+        a[i] = cat8(lds_ld128(sa_ + r * 128 + ((g ^ wide_swz(wm + r)) * 16)),
+                    lds_ld128(sa_ + r * 128 + (((g + 4) ^ wide_swz(wm + r)) * 16)));
+        w[i] = cat8(lds_ld128(sw_ + r * 128 + ((g ^ wide_swz(wn + r)) * 16)),
+                    lds_ld128(sw_ + r * 128 + (((g + 4) ^ wide_swz(wn + r)) * 16)));
+      }
+#pragma unroll
+      for (int ms = 0; ms < 2; ++ms)
+#pragma unroll
+        for (int ns = 0; ns < 2; ++ns) {
+          if constexpr (FMT == kE5M2A)  // W e4m3 (format 0), A e5m2 (format 1)
+            acc4[ms][ns] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w[ns], a[ms], acc4[ms][ns], 0, 1, 0, 0, 0, 0);
+          else
+            acc4[ms][ns] = mfma_fp8(w[ns], a[ms], acc4[ms][ns]);
+        }
+    }
+  };
+  for (int s = 0; s < nk - 2; ++s) kstep(s, std::integral_constant<int, 8>{});
+  if (nk >= 2) kstep(nk - 2, std::integral_constant<int, 4>{});
+  kstep(nk - 1, std::integral_constant<int, 0>{});
+
+  // rows past M: stores are dropped, residual loads read zero (range check)
+  constexpr int ES = E4M3_OUT ? 1 : 2;
+  const BufRsrc crs = make_rsrc((uint8_t*)p.C + (int64_t)m0 * p.ldc * ES, (uint32_t)(mrows * p.ldc * ES));
+  const BufRsrc rrs = make_rsrc(RESID ? (const void*)(p.resid + (int64_t)m0 * p.ldr) : p.C,
+                                RESID ? (uint32_t)(mrows * p.ldr * 2) : 0u);
+  const bool silu = n0 + wn >= p.silu_begin && n0 + wn < p.silu_end;
+  const float os = E4M3_OUT ? p.out_scale[0] : 1.f;
+  const float oy = E4M3_OUT ? 1.f / os : 1.f;
+#pragma unroll
+  for (int run = 0; run < 2; ++run) {  // fp8: row block, bf16: column run
+    const int r = FMT == kBF16 ? wm + lr : wm + 16 * run + li;
+    const int c = FMT == kBF16 ? c0 + 16 * run : c0;
+    const u32x4 b = FMT == kBF16 ? bv[run] : bv[0];
+    float o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t bw = b[e >> 1];
+      const float bb = bf16_to_f32((uint16_t)(e & 1 ? bw >> 16 : bw & 0xffff));
+      if constexpr (FMT == kBF16) {
+        o[e] = acc16[8 * run + e] + bb;
+      } else {
+        const float a = acc4[run][e >> 2][e & 3], sc = sa[run] * sw[e >> 2][e & 3];
+        o[e] = E4M3_OUT ? mul_then_add(a, sc, bb) : a * sc + bb;
+      }
+    }
+    if (silu) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = o[e] * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-kLog2e * o[e]));
+    }
+    if constexpr (RESID) {
+      const u32x4 rv = buf_ld128(rrs, (uint32_t)(r * p.ldr + c) * 2, 0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        o[2 * j] += bf16_to_f32((uint16_t)(rv[j] & 0xffff));
+        o[2 * j + 1] += bf16_to_f32((uint16_t)(rv[j] >> 16));
+      }
+    }
+    if constexpr (E4M3_OUT) {
+      float q[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        q[e] = __builtin_fminf(__builtin_fmaxf(os == 1.f ? o[e] : div_by(o[e], os, oy), -448.f), 448.f);
+      const uint32_t w0 = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false), true);
+      const uint32_t w1 = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(q[6], q[7], __builtin_amdgcn_cvt_pk_fp8_f32(q[4], q[5], 0, false), true);
+      __builtin_amdgcn_raw_buffer_store_b64(u32x2{w0, w1}, crs, (uint32_t)(r * p.ldc + c), 0, 0);
+    } else {
+      __builtin_amdgcn_raw_buffer_store_b128(
+          u32x4{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3]), pack_bf16(o[4], o[5]), pack_bf16(o[6], o[7])}, crs,
+          (uint32_t)(r * p.ldc + c) * 2, 0, 0);
+    }
   }
 }
 
@@ -1640,6 +1828,23 @@ hipError_t set_gemm_lds(const void* fn) {
   return e;
 }
 
+// The few-row form serves products of at most 80 wide (128 x 256) tiles: its
+// 640 tiles are 1.25 rounds of the chip's 512 workgroup slots.  Measured on
+// both sides of the line (us, few-row / wide): bf16 [4 000, 2048] x [2048, 512]
+// (64 wide tiles) 21.6 / 29.0, [8 000, 2048] (126) 39.6 / 30.0; e4m3
+// [4 000, 1536] x [1536, 512] 11.5 / 16.9, [8 000, 1536] 19.9 / 18.2;
+// [1 027, 512] x [512, 2048] (72) bf16 8.2 / 11.5, e4m3 5.8 / 8.6, [4 000, 512]
+// (256) 22.8 / 15.4, 12.0 / 10.7.
+constexpr int kFewMaxWideTiles = 80;
+bool few_rows(int M, int N) { return (int64_t)((M + kBM - 1) / kBM) * (N / kWideBN) <= kFewMaxWideTiles; }
+int launch_few_rows(void (*kern)(GemmParams), GemmParams p, hipStream_t stream) {
+  p.tiles_m = (p.M + kFewB - 1) / kFewB;
+  p.tiles_n = p.N / kFewB;
+  const int per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
+  void* args[] = {&p};
+  return (int)hipLaunchKernel((const void*)kern, dim3(8 * per_xcd), dim3(kThreads), args, 0, stream);
+}
+
 }  // namespace
 
 extern "C" int hstu_fp8_gemm(int a_dtype, const void* A, int64_t lda, const void* W, int64_t ldw,
@@ -1688,6 +1893,13 @@ extern "C" int hstu_fp8_gemm(int a_dtype, const void* A, int64_t lda, const void
       (int64_t)M * 4 <= 0xffffffffLL &&
       (!residual || ((uintptr_t)residual % 16 == 0 && ldr % 8 == 0)) && (int64_t)(N - 1) * ldw + K <= 0xffffffffLL &&
       (a_dtype == HSTU_DTYPE_FP8_E4M3 || (!out8 && !residual));
+  if (wide_ok && few_rows(M, N)) {  // the same bytes as the forms below
+    void (*fk)(GemmParams);
+    if (a_dtype == HSTU_DTYPE_FP8_E5M2) fk = gemm_few_rows_kernel<false, false, kE5M2A>;
+    else if (out8) fk = residual ? gemm_few_rows_kernel<true, true, kE4M3> : gemm_few_rows_kernel<true, false, kE4M3>;
+    else fk = residual ? gemm_few_rows_kernel<false, true, kE4M3> : gemm_few_rows_kernel<false, false, kE4M3>;
+    return launch_few_rows(fk, p, stream);
+  }
   if (wide_ok) {
     p.tiles_n = N / kWideBN;
     const int total = p.tiles_m * p.tiles_n;
@@ -1772,14 +1984,18 @@ extern "C" int hstu_bf16_gemm(const void* A, int64_t lda, const void* W, int64_t
   p.silu_begin = silu_begin;
   p.silu_end = silu_end;
   p.tiles_m = (M + kBM - 1) / kBM;
-  // two-workgroup form: whole 256-column tiles, at least two k-steps, 16-byte
-  // output and residual rows, a SiLU range of whole waves (64 columns).  The
-  // rule does not look at M, so a row's bytes do not depend on its batch.
+  // two-workgroup form (few rows: the few-row form, the same MFMA chain):
+  // whole 256-column tiles, at least two k-steps, 16-byte output and residual
+  // rows, a SiLU range of whole waves (64 columns).  duo_ok does not look at M,
+  // so a row's bytes do not depend on its batch.
   const bool duo_ok = N % kWideBN == 0 && p.K >= 2 * kBK && (uintptr_t)C % 16 == 0 && ldc % 8 == 0 &&
                       (!residual || ((uintptr_t)residual % 16 == 0 && ldr % 8 == 0)) &&
                       (silu_begin >= silu_end || (silu_begin % 64 == 0 && silu_end % 64 == 0)) &&
                       (int64_t)kBM * 2 * ldc <= 0xffffffffLL && (int64_t)kBM * 2 * ldr <= 0xffffffffLL &&
                       (int64_t)(kWideBN - 1) * p.ldw + p.K <= 0xffffffffLL;
+  if (duo_ok && few_rows(M, N))
+    return launch_few_rows(residual ? gemm_few_rows_kernel<false, true, kBF16> : gemm_few_rows_kernel<false, false, kBF16>,
+                           p, stream);
   if (duo_ok) {
     p.tiles_n = N / kWideBN;
     int per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;

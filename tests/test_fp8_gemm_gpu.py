@@ -338,3 +338,32 @@ def test_bf16_gemm_two_workgroup_form(hip_lib, M, N, K, resid, pad):
         ref = ref + r.double()
     assert orc.rel_l2(ref, wide[:, :N].cpu().double()) <= 4e-3
     assert bool((wide[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("fmt,N,K,resid,out8", [("bf16", 512, 128, False, False), ("bf16", 512, 1536, True, False),
+                                                ("e4m3", 512, 1536, True, False), ("e4m3", 768, 256, False, True),
+                                                ("e4m3", 256, 512, True, True), ("e4m3", 2048, 512, False, False)])
+def test_gemm_few_row_form_same_bytes(hip_lib, fmt, N, K, resid, out8):
+    """The few-row form gives the bytes of the wide forms: 1, 64, 65 and 300
+    rows of a product large enough for the wide form, computed alone."""
+    fp8 = _fp8()
+    g = torch.Generator().manual_seed(N + K)
+    M = 128 * (81 * 256 // N + 1)
+    a = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = torch.randn(N, K, generator=g) / K ** 0.5
+    b = None if resid else (0.1 * torch.randn(N, generator=g)).to(torch.bfloat16).to(DEV)
+    r = torch.randn(M, N, generator=g).to(torch.bfloat16).to(DEV) if resid else None
+    if fmt == "bf16":
+        ad, wd = a.to(DEV), w.to(torch.bfloat16).to(DEV)
+        run = lambda s: fp8.bf16_gemm(ad[s], wd, bias=b, residual=None if r is None else r[s])  # noqa: E731
+    else:
+        a8, sa = fp8.quantize_e4m3_rows(a.to(DEV))
+        wt = fp8.quantize_weight_e4m3(w.to(torch.bfloat16).t().contiguous().to(DEV))
+        kw = dict(out_dtype=torch.float8_e4m3fn, out_scale=torch.tensor([0.01], device=DEV)) if out8 else {}
+        run = lambda s: fp8.fp8_gemm(a8[s], sa.reshape(-1)[s], wt, bias=b,  # noqa: E731
+                                     residual=None if r is None else r[s],
+                                     silu_cols=None if out8 else (64, 192), **kw)
+    full = run(slice(0, M)).view(torch.uint8)
+    for rows in (1, 64, 65, 300):
+        s = slice(200, 200 + rows)
+        assert torch.equal(full[s], run(s).view(torch.uint8)), rows
