@@ -340,13 +340,7 @@ __device__ __forceinline__ uint8_t* ds_tile(const AttnParams& p, const SeqCtx& c
 }
 
 __device__ __forceinline__ MaskCtx mask_ctx(const AttnParams& p, const SeqCtx& c) {
-  MaskCtx m;
-  m.L = c.L;
-  m.targets = p.num_targets != nullptr;
-  m.nt = m.targets ? p.num_targets[c.b] : 0;
-  m.ctx = p.contextual_seq_len;
-  m.max_attn = p.max_attn_len;
-  return m;
+  return mask_make(c.L, p.num_targets, c.b, p.max_attn_len, p.contextual_seq_len);
 }
 
 // =====================================================================
@@ -483,8 +477,13 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt) o[qt][dt] = zero4();
 
-  int n_end = min(m0 + C::BM, L);
-  if (GENERIC && m0 < p.contextual_seq_len) n_end = L;
+  // key tiles t_begin .. ntiles - 1: generic masks skip the keys outside the
+  // window, and a block with prefix rows sees the whole sequence
+  int n_end = min(m0 + C::BM, L), t_begin = 0;
+  if constexpr (GENERIC) {
+    if (m0 < p.contextual_seq_len) n_end = L;
+    else t_begin = mask_first_key(m0, mc) / C::BN;
+  }
   const int ntiles = (n_end + C::BN - 1) / C::BN;
 
   FwdStage<D, FP8> stg;
@@ -556,16 +555,25 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
   // bias index of element (qt, kt, r) = bias_rd + 16*(qt-kt) - r
   const int bias_rd = 32 * wave + (C::BN - 1) + li - 4 * g;
 
-  load(0);
-  store(smem);
+  // positions of the lane's queries (generic masks)
+  int qid[2] = {0, 0};
+  if constexpr (GENERIC) {
+    qid[0] = mask_id(mw0 + li, mc);
+    qid[1] = mask_id(mw0 + 16 + li, mc);
+  }
+
+  load(t_begin * C::BN);
+  store(smem + (t_begin & 1) * C::BUF);
   __syncthreads();
 
-  for (int t = 0; t < ntiles; ++t) {
+  for (int t = t_begin; t < ntiles; ++t) {
     const int n0 = t * C::BN;
     const uint8_t* buf = smem + (t & 1) * C::BUF;
     if (t + 1 < ntiles) load(n0 + C::BN);
 
-    if (wave_active && (GENERIC || n0 <= mw0 + 31)) {
+    const MaskClass cls = GENERIC ? mask_class(mw0, mw0 + 31, n0, n0 + C::BN - 1, mc)
+                                  : n0 > mw0 + 31 ? kMaskNone : n0 + C::BN - 1 > mw0 ? kMaskSome : kMaskAll;
+    if (wave_active && cls != kMaskNone) {
       // ---- S^T = K . Q^T : s[kt][qt], keys n0+16kt+4g+r, query mw0+16qt+li
       f32x4 s[C::KT][2];
 #pragma unroll
@@ -588,7 +596,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
         }
       }
       // ---- SiLU epilogue on the accumulators, packed into P (A operand)
-      const bool need_mask = GENERIC || (n0 + C::BN - 1 > mw0);
+      const bool need_mask = cls == kMaskSome;
       // whole tile in the clamped bias region: one constant
       const bool bias_const = BIAS && (m0 - n0 - (C::BN - 1) >= R1);
       const float* bias_lds = (const float*)(buf + C::BIAS_OFF);
@@ -620,7 +628,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
               else val = t * sig_of_t(t);
               if constexpr (MASKED) {
                 const int i = mw0 + qt * 16 + li, j = n0 + kt * 16 + 4 * g + r;
-                const bool ok = GENERIC ? valid_generic(i, j, mc) : (j <= i);
+                const bool ok = GENERIC ? mask_pair(i, j, qid[qt], mask_id(j, mc), mc) : (j <= i);
                 val = ok ? val : 0.f;
               }
               pv[r] = val;
@@ -1320,7 +1328,8 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
   if (m0 >= L) return;
   const MaskCtx mc = mask_ctx(p, sc);
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15,
+            g = lane >> 4;
   const int mw0 = m0 + wave * 32;
   const bool wave_active = mw0 < L;
 
@@ -1365,9 +1374,17 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt) acc[qt][dt] = zero4();
 
-  int n_end = min(m0 + C::BM, L);
-  if (GENERIC && m0 < p.contextual_seq_len) n_end = L;
+  int n_end = min(m0 + C::BM, L), t_begin = 0;  // as in the forward
+  if constexpr (GENERIC) {
+    if (m0 < p.contextual_seq_len) n_end = L;
+    else t_begin = mask_first_key(m0, mc) / C::BN;
+  }
   const int ntiles = (n_end + C::BN - 1) / C::BN;
+  int qid[2] = {0, 0};
+  if constexpr (GENERIC) {
+    qid[0] = mask_id(mw0 + li, mc);
+    qid[1] = mask_id(mw0 + 16 + li, mc);
+  }
 
   RowStage<C::BN, D, FP8> k_st, v_st;
   k_st.init(krs, C::K_OFF);
@@ -1404,17 +1421,19 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
   const int bias_rd = 32 * wave + (C::BN - 1) + li - 4 * g;
   float dclamp = 0.f, dclampn = 0.f;  // bias gradient of elements in the clamped regions (+, -)
 
-  load(0);
-  store(smem);
+  load(t_begin * C::BN);
+  store(smem + (t_begin & 1) * C::BUF);
   __syncthreads();
 
-  for (int t = 0; t < ntiles; ++t) {
+  for (int t = t_begin; t < ntiles; ++t) {
     const int n0 = t * C::BN;
     const uint8_t* buf = smem + (t & 1) * C::BUF;
     if (t + 1 < ntiles) load(n0 + C::BN);
 
-    if (wave_active && (GENERIC || n0 <= mw0 + 31)) {
-      const bool need_mask = GENERIC || (n0 + C::BN - 1 > mw0);
+    const MaskClass cls = GENERIC ? mask_class(mw0, mw0 + 31, n0, n0 + C::BN - 1, mc)
+                                  : n0 > mw0 + 31 ? kMaskNone : n0 + C::BN - 1 > mw0 ? kMaskSome : kMaskAll;
+    if (wave_active && cls != kMaskNone) {
+      const bool need_mask = cls == kMaskSome;
       const bool bias_const = BIAS && (m0 - n0 - (C::BN - 1) >= R1);
       const float* bias_lds = (const float*)(buf + C::BIAS_OFF);
       // Two halves of 32 keys each (key sub-tiles 2c, 2c+1), to keep the
@@ -1464,7 +1483,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
                 float ds = dsilu_dp(t, FP8 ? dp[h2][qt][r] * svv[r] : dp[h2][qt][r]);
                 if constexpr (MASKED) {
                   const int i = mw0 + qt * 16 + li, j = n0 + kt * 16 + 4 * g + r;
-                  const bool ok = GENERIC ? valid_generic(i, j, mc) : (j <= i);
+                  const bool ok = GENERIC ? mask_pair(i, j, qid[qt], mask_id(j, mc), mc) : (j <= i);
                   ds = ok ? ds : 0.f;
                 }
                 if constexpr (BIAS) {
@@ -1844,7 +1863,8 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
   if (n0 >= L) return;
   const MaskCtx mc = mask_ctx(p, sc);
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15,
+            g = lane >> 4;
   const int kw0 = n0 + wave * 32;
   const bool wave_active = kw0 < L;
 
@@ -1905,8 +1925,15 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt) dk[kt][dt] = dv[kt][dt] = zero4();
 
-  const int m_begin = GENERIC ? 0 : n0;
-  const int ntiles = (L - m_begin + C::BMQ - 1) / C::BMQ;
+  // Query tiles, in order: with a contextual prefix its rows (which see every
+  // history key), then rows n0 up to the last one inside the window.
+  int npre = 0, m_end = L;
+  if constexpr (GENERIC) {
+    npre = min((p.contextual_seq_len + C::BMQ - 1) / C::BMQ, n0 / C::BMQ);
+    m_end = max(mask_end_row(min(n0 + C::BN, L) - 1, L, mc), n0 + 1);
+  }
+  const int ntiles = npre + (m_end - n0 + C::BMQ - 1) / C::BMQ;
+  auto tile_m0 = [&](int t) { return GENERIC && t < npre ? t * C::BMQ : n0 + (t - npre) * C::BMQ; };
 
   // Per-lane global offset of load instruction i of a tile of padded rows
   // (cpr 16-byte slots per LDS row, dcpr of them data); recomputed at each
@@ -1989,7 +2016,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
   const int R1 = p.bias_R - 1;
 
 #pragma unroll
-  for (int st = 0; st < C::NSTAGE - 1; ++st) issue(m_begin + st * C::BMQ, smem + st * C::STAGE);
+  for (int st = 0; st < C::NSTAGE - 1; ++st) issue(tile_m0(st), smem + st * C::STAGE);
   wait_vm_le<(C::NSTAGE - 2) * C::CNT>();
   __syncthreads();
 
@@ -2001,16 +2028,18 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
   auto tile_body = [&](int t, auto masked_tag, auto bconst_tag) {
     constexpr bool MASKED = decltype(masked_tag)::value;
     constexpr bool BCONST = decltype(bconst_tag)::value;
-    const int m0 = m_begin + t * C::BMQ;
+    const int m0 = tile_m0(t);
     const uint8_t* buf = smem + cur * C::STAGE;
     {
       int nxt = cur + C::NSTAGE - 1;
       nxt = nxt >= C::NSTAGE ? nxt - C::NSTAGE : nxt;
-      issue(m0 + (C::NSTAGE - 1) * C::BMQ, smem + nxt * C::STAGE);
+      issue(tile_m0(t + C::NSTAGE - 1), smem + nxt * C::STAGE);
     }
 
     u32x4 ds_out[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};  // this tile's dS for the dQ kernel
-    if (wave_active && (GENERIC || m0 + C::BMQ - 1 >= kw0)) {
+    const bool any = !GENERIC ? m0 + C::BMQ - 1 >= kw0
+                              : !MASKED || mask_class(m0, m0 + C::BMQ - 1, kw0, kw0 + 31, mc) != kMaskNone;
+    if (wave_active && any) {
       f32x4 s[C::QS][2], dp[C::QS][2];
 #pragma unroll
       for (int qs = 0; qs < C::QS; ++qs) {
@@ -2055,7 +2084,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
             if constexpr (FP8) dval *= sqv[r];
             if constexpr (MASKED) {
               const int i = m0 + qs * 16 + 4 * g + r, j = kw0 + kt * 16 + li;
-              const bool ok = GENERIC ? valid_generic(i, j, mc) : (j <= i);
+              const bool ok = GENERIC ? mask_pair(i, j, mask_id(i, mc), mask_id(j, mc), mc) : (j <= i);
               pval = ok ? pval : 0.f;
               dval = ok ? dval : 0.f;
             }
@@ -2106,17 +2135,29 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
     }
   };
 
-  // Tiles [0, t_mask) touch the diagonal of some wave's keys (queries below
-  // n0 + BN - 1); tiles from t_const on have every offset i-j >= R-1 and so a
-  // constant bias.
-  const int t_mask = GENERIC ? ntiles : min(ntiles, (C::BN - 1 + C::BMQ - 1) / C::BMQ);
-  int t_const = ntiles;
-  if (BIAS && !GENERIC) t_const = max(t_mask, min(ntiles, (R1 + C::BN - 1 + C::BMQ - 1) / C::BMQ));
   int t = 0;
-  for (; t < t_mask; ++t) tile_body(t, std::true_type{}, std::false_type{});
-  for (; t < t_const; ++t) tile_body(t, std::false_type{}, std::false_type{});
-  if constexpr (BIAS) {
-    for (; t < ntiles; ++t) tile_body(t, std::false_type{}, std::true_type{});
+  if constexpr (GENERIC) {
+    // masked tiles (prefix, diagonal), the run of tiles whose pairs are all
+    // valid, then the rest masked (the window's edge)
+    auto all = [&](int u) {
+      const int m0 = tile_m0(u);
+      return mask_class(m0, m0 + C::BMQ - 1, n0, n0 + C::BN - 1, mc) == kMaskAll;
+    };
+    for (; t < ntiles && !all(t); ++t) tile_body(t, std::true_type{}, std::false_type{});
+    for (; t < ntiles && all(t); ++t) tile_body(t, std::false_type{}, std::false_type{});
+    for (; t < ntiles; ++t) tile_body(t, std::true_type{}, std::false_type{});
+  } else {
+    // Tiles [0, t_mask) touch the diagonal of some wave's keys (queries below
+    // n0 + BN - 1); tiles from t_const on have every offset i-j >= R-1 and so a
+    // constant bias.
+    const int t_mask = min(ntiles, (C::BN - 1 + C::BMQ - 1) / C::BMQ);
+    int t_const = ntiles;
+    if (BIAS) t_const = max(t_mask, min(ntiles, (R1 + C::BN - 1 + C::BMQ - 1) / C::BMQ));
+    for (; t < t_mask; ++t) tile_body(t, std::true_type{}, std::false_type{});
+    for (; t < t_const; ++t) tile_body(t, std::false_type{}, std::false_type{});
+    if constexpr (BIAS) {
+      for (; t < ntiles; ++t) tile_body(t, std::false_type{}, std::true_type{});
+    }
   }
 
   if (!wave_active) return;

@@ -4,6 +4,7 @@
 #define HSTU_COMMON_H_
 
 #include <hip/hip_runtime.h>
+#include <climits>
 #include <utility>
 #include <stdint.h>
 
@@ -271,28 +272,56 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // ---------------------------------------------------------------- mask
+// _get_valid_attn_mask (ops/pytorch/pt_hstu_attention.py:32-84) in terms of
+// the position id(x) = min(max(x - c1, 0), clamp), nondecreasing in x: the
+// contextual prefix shares position 0 and the targets share the last one.
+// Pair (i, j) is valid when i == j, when 0 < id(i) - id(j) <= window, or when
+// i is a prefix row (position 0) and j a history key (id(j) < last).
 struct MaskCtx {
-  int L, nt, ctx, max_attn;
-  bool targets;
+  int c1;      // contextual_seq_len - 1, or 0 without a prefix
+  int clamp;   // position of the targets, INT_MAX without targets
+  int window;  // max_attn_len, INT_MAX without
+  int last;    // prefix rows see keys of positions below this (0 without a prefix: none)
 };
-// _get_valid_attn_mask (ops/pytorch/pt_hstu_attention.py:32-84), per element.
-__device__ __forceinline__ bool valid_generic(int i, int j, const MaskCtx& m) {
-  int max_ids = m.L, ii = i, jj = j;
-  if (m.ctx > 0) {
-    ii = max(i - m.ctx + 1, 0);
-    jj = max(j - m.ctx + 1, 0);
-    max_ids = m.L - m.ctx + 1;
-  }
-  if (m.targets) {
-    max_ids -= m.nt;
-    ii = min(ii, max_ids);
-    jj = min(jj, max_ids);
-  }
-  const int dist = ii - jj;
-  bool v = (i == j) || (dist > 0);
-  if (m.max_attn > 0) v = v && (dist <= m.max_attn);
-  if (m.ctx > 0) v = v || (ii == 0 && jj < max_ids);
-  return v && j < m.L && i < m.L;
+__device__ __forceinline__ MaskCtx mask_make(int L, const int32_t* num_targets, int b, int max_attn_len, int ctx) {
+  MaskCtx m;
+  m.c1 = ctx > 0 ? ctx - 1 : 0;
+  const int last = L - m.c1 - (num_targets ? num_targets[b] : 0);
+  m.clamp = num_targets ? last : INT_MAX;
+  m.window = max_attn_len > 0 ? max_attn_len : INT_MAX;
+  m.last = ctx > 0 ? last : INT_MIN;
+  return m;
+}
+__device__ __forceinline__ int mask_id(int x, const MaskCtx& m) { return min(max(x - m.c1, 0), m.clamp); }
+// The mask of a pair with positions a = id(i), b = id(j).
+__device__ __forceinline__ bool mask_pair(int i, int j, int a, int b, const MaskCtx& m) {
+  return (i == j) | ((unsigned)(a - b - 1) < (unsigned)m.window) | ((a == 0) & (b < m.last));
+}
+// What the mask leaves of rows i0 .. i1 against keys j0 .. j1: kMaskNone only
+// if no pair is valid, kMaskAll only if every pair is (then j1 < i0, so no
+// key is past the sequence; rows past it read as zero and are not stored).
+// Testing every element of every tile was what bounded the kernels with these
+// masks: 64 sequences of 128 .. 1024, window 256, targets and a prefix, bf16,
+// forward + backward 543 -> 251 us; one sequence of 3 001 with targets, forward
+// 234 -> 80 us.
+enum MaskClass { kMaskNone = 0, kMaskSome = 1, kMaskAll = 2 };
+__device__ __forceinline__ MaskClass mask_class(int i0, int i1, int j0, int j1, const MaskCtx& m) {
+  const int a0 = mask_id(i0, m), a1 = mask_id(i1, m), b0 = mask_id(j0, m), b1 = mask_id(j1, m);
+  if (a0 > b1 && a1 - b0 <= m.window) return kMaskAll;
+  const bool diag = i0 <= j1 && j0 <= i1;
+  const bool near = a1 > b0 && a0 - b1 <= m.window;
+  const bool prefix = a0 == 0 && b0 < m.last;
+  return diag || near || prefix ? kMaskSome : kMaskNone;
+}
+// First key a row block starting at row m0 (no prefix row) can see.
+__device__ __forceinline__ int mask_first_key(int m0, const MaskCtx& m) {
+  const int a = mask_id(m0, m);
+  return m.window < a ? a - m.window + m.c1 : 0;
+}
+// One past the last row (of L) that sees a key block ending at key n1.
+__device__ __forceinline__ int mask_end_row(int n1, int L, const MaskCtx& m) {
+  const int b = mask_id(n1, m);
+  return m.window < m.clamp - b && m.window < L - b - m.c1 ? b + m.window + m.c1 + 1 : L;
 }
 
 // vmcnt(0); expcnt and lgkmcnt left at their maxima.

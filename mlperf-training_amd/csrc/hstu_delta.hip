@@ -96,13 +96,7 @@ __device__ __forceinline__ DeltaSeq delta_seq(const DeltaParams& p, int b) {
   return s;
 }
 __device__ __forceinline__ MaskCtx delta_mask(const DeltaParams& p, const DeltaSeq& s) {
-  MaskCtx m;
-  m.L = s.L;
-  m.targets = p.num_targets != nullptr;
-  m.nt = m.targets ? p.num_targets[s.b] : 0;
-  m.ctx = p.contextual_seq_len;
-  m.max_attn = p.max_attn_len;
-  return m;
+  return mask_make(s.L, p.num_targets, s.b, p.max_attn_len, p.contextual_seq_len);
 }
 
 // ------------------------------------------------------------------ layout
@@ -248,7 +242,7 @@ __global__ void __launch_bounds__(kThreads) delta_fwd_kernel(DeltaParams p) {
       const float x = group_sum<M::LPR>(part) * xs;
       const int jj = (t + u) * M::RPB + slot;
       float w = 0.f;
-      if (jj < jn && i >= 0 && valid_generic(i, j0 + jj, mc))
+      if (jj < jn && i >= 0 && mask_pair(i, j0 + jj, mask_id(i, mc), mask_id(j0 + jj, mc), mc))
         w = x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-kLog2e * x)) * p.inv_n;
       wb[u] = to_bf16(w);
     }
@@ -417,7 +411,7 @@ __global__ void __launch_bounds__(kThreads) delta_bwd_kernel(DeltaParams p) {
         const float dpv = group_sum<M::LPR>(dpp);
         const int i = sq.L - DS + r;
         w[r] = ds[r] = 0.f;
-        if (jj < jl && i >= 0 && valid_generic(i, j0 + jj, mc)) {
+        if (jj < jl && i >= 0 && mask_pair(i, j0 + jj, mask_id(i, mc), mask_id(j0 + jj, mc), mc)) {
           const float sg = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-kLog2e * x));
           w[r] = bf16_round(x * sg * p.inv_n);
           ds[r] = bf16_round(dpv * sg * (1.f + x * (1.f - sg)) * p.inv_n);

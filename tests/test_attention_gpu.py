@@ -145,6 +145,40 @@ def test_generic_masks(hip_lib, mode):
         _check_bf16(got.float().cpu() / s, r / s, f"{name} {mode}")
 
 
+@pytest.mark.parametrize("win,ctx,nts,D,with_bias", [
+    (1, 0, None, 64, False), (63, 0, None, 128, True), (64, 0, [0, 64, 500, 1], 128, False),
+    (65, 33, None, 64, True), (200, 130, [7, 64, 3, 1], 128, True), (0, 129, [200, 0, 2, 1], 64, False),
+    (0, 0, [130, 65, 300, 1], 128, True), (31, 2, [1, 128, 33, 2], 128, False)])
+def test_generic_mask_tiles(hip_lib, win, ctx, nts, D, with_bias):
+    """Windows, prefixes and targets around the tile sizes (32, 64, 128), so
+    that tiles are skipped, taken whole and cut: forward, dq, dk, dv and the
+    bias gradient at the bf16 bar (the bias gradient at relative L2 <= 1e-2)."""
+    ops = _ops()
+    lengths = [385, 129, 257, 3]
+    H, N = 2, 400
+    q, k, v, offs = _case(lengths, H, D, seed=win + ctx)
+    nt = None if nts is None else torch.tensor(nts, dtype=torch.int64)
+    bias = orc.make_bias(H, 100, seed=2, std=0.3) if with_bias else None
+    alpha = 0.15
+    qd, kd, vd = (t.to(DEV).requires_grad_(True) for t in (q, k, v))
+    bd = None if bias is None else bias.to(DEV).requires_grad_(True)
+    out = ops.triton_hstu_mha(N, alpha, qd, kd, vd, offs.to(DEV), None if nt is None else nt.to(DEV), win, ctx,
+                              attn_bias=bd)
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
+    out.backward(dout.to(DEV))
+    torch.cuda.synchronize()
+    ref = orc.hstu_mha_dense(N, alpha, q.double(), k.double(), v.double(), offs, nt, win, ctx,
+                             None if bias is None else bias.double(), dtype=torch.float64)
+    scale = ref.abs().max()
+    _check_bf16(out.detach().float().cpu() / scale, ref / scale, "fwd")
+    dq, dk, dv, db = orc.hstu_mha_bwd(N, alpha, q, k, v, offs, dout, nt, win, ctx, bias)
+    for name, got, r in (("dq", qd.grad, dq), ("dk", kd.grad, dk), ("dv", vd.grad, dv)):
+        s = r.abs().max()
+        _check_bf16(got.float().cpu() / s, r / s, name)
+    if bias is not None:
+        assert orc.rel_l2(db, bd.grad.double().cpu()) <= 1e-2
+
+
 def test_strided_uvqk_views(hip_lib):
     """q/k/v read in place as column slices of a fused [T, 2048] buffer, and
     dq/dk/dv written into strided views of a fused gradient buffer."""
