@@ -231,13 +231,12 @@ struct AttnParams {
   float* dbias_part;      // workspace: one bias-gradient row per dQ block [blocks, H, dbias_w]
   const int64_t* dq_base;  // workspace: per-sequence exclusive prefix of 128-query blocks [B + 1]
   int dbias_w;            // floats per row: offsets 0 .. R-1 (causal), -(R-1) .. R-1 (generic masks)
-  const int* sched_items;  // block schedule (schedule_block): [8][sched_cap] (sequence*H + head)
+  const int* sched_items;  // block schedule (schedule_block): [8][sched_cap] (sequence*H + head); null: direct grid
   const int* sched_start;  // [8][sched_cap + 1] first block position of each item on its XCD
   const int* sched_count;  // [8] items per XCD
   int sched_cap;
   int blocks_per_seq;  // ceil(N / 128)
   uint8_t* ds_ws;           // workspace: bf16 dS tiles written by dK/dV, read by dQ (causal masks)
-  const int64_t* ds_base;   // workspace: per-sequence exclusive prefix of ds_tiles(L) [B + 1]
   // full-FP8 backward (hstu_attn_bwd_fp8)
   const uint8_t* do8;       // e4m3 dO [T, H, D], row stride do_rs bytes
   const uint8_t* e8;        // [T, H]: 127 - e of each token's dO group (dO8 = e4m3(dO * 2^e))
@@ -288,42 +287,64 @@ __device__ __forceinline__ void dbias_store_row(const AttnParams& p, const float
 struct SeqCtx {
   int64_t start;
   int L, b, h, blk;
+  int tail;  // direct grid, first block of an item: rows past N that the item's outputs must zero
 };
-// Workgroup -> (sequence, head, 128-row block), from the schedule that
-// schedule_block wrote: workgroup i runs on XCD x = i % 8 and takes the
-// (i / 8)-th block of that XCD's list.  heavy_last: the block with the most
-// key tiles is the last one of its sequence (forward, dQ) rather than the
+// Workgroup -> (sequence, head, 128-row block).  heavy_last: the block with the
+// most key tiles is the last one of its sequence (forward, dQ) rather than the
 // first (dK/dV); each item's blocks run heaviest first.  False = no work.
 // With half != nullptr two workgroups share each block (i = 16 k + 8 h + x:
 // half h of the k-th block), on the same XCD one after the other.
+//  * scheduled: from what schedule_block wrote; workgroup i runs on XCD
+//    x = i % 8 and takes the (i / 8)-th block of that XCD's list.
+//  * direct (no schedule): block m of item u % (B H), m = u / (B H), u the
+//    workgroup (pair), so all items' heaviest blocks come first and one item's
+//    blocks spread over the XCDs when there are few items.
 __device__ __forceinline__ bool seq_ctx(const AttnParams& p, bool heavy_last, SeqCtx& c, int* half = nullptr) {
   const int x = blockIdx.x & 7, k = half ? blockIdx.x >> 4 : blockIdx.x >> 3;
   if (half) *half = (blockIdx.x >> 3) & 1;
-  const int n = p.sched_count[x];
-  const int* st = p.sched_start + x * (p.sched_cap + 1);
-  if (k >= st[n]) return false;
-  int lo = 0, hi = n - 1;  // the last item whose first block is <= k
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (st[mid] <= k) lo = mid;
-    else hi = mid - 1;
+  int bh, m;
+  if (p.sched_items == nullptr) {
+    const int u = 8 * k + x, items = p.B * p.H;
+    m = u / items;
+    bh = u - m * items;
+  } else {
+    const int n = p.sched_count[x];
+    const int* st = p.sched_start + x * (p.sched_cap + 1);
+    if (k >= st[n]) return false;
+    int lo = 0, hi = n - 1;  // the last item whose first block is <= k
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (st[mid] <= k) lo = mid;
+      else hi = mid - 1;
+    }
+    bh = p.sched_items[x * p.sched_cap + lo];
+    m = k - st[lo];
   }
-  const int bh = p.sched_items[x * p.sched_cap + lo];
-  const int m = k - st[lo];
   c.b = bh / p.H;
   c.h = bh - c.b * p.H;
   c.start = p.seq_offsets[c.b];
-  c.L = min((int)(p.seq_offsets[c.b + 1] - c.start), p.N);
+  const int64_t len = p.seq_offsets[c.b + 1] - c.start;
+  c.L = min((int)len, p.N);
   const int nb = (c.L + 127) / 128;
   c.blk = heavy_last ? nb - 1 - m : m;
-  return true;
+  c.tail = p.sched_items == nullptr && m == 0 ? (int)len - c.L : 0;
+  return m < nb;
+}
+// Zeroes columns h D .. h D + D - 1 of rows N .. N + tail - 1 of a sequence's
+// output (the set-up launch does it when there is a schedule).
+template <int D>
+__device__ __forceinline__ void zero_tail(const SeqCtx& c, int N, uint16_t* out, int64_t rs) {
+  for (int i = threadIdx.x; i < c.tail * D; i += blockDim.x) out[(c.start + N + i / D) * rs + (int64_t)c.h * D + i % D] = 0;
 }
 // dS tiles.  For the causal mask the dK/dV kernel computes dS for key block
 // kb (128 keys) against query tiles qt = 4 kb .. ceil(L/32) - 1 (32 queries);
 // it stores each such (kb, qt) tile, bf16, for the dQ kernel to contract
 // with K instead of recomputing S, dP and the SiLU derivative.  Tiles of one
 // (sequence, head) are consecutive in kb-major order, so tile (kb, qt) is at
-// kb * QT - 2 kb^2 - 2 kb + qt, and a sequence has ds_tiles(L) of them.
+// kb * QT - 2 kb^2 - 2 kb + qt, and a sequence has ds_tiles(L) of them.  A
+// sequence's tiles start at 2 (ceil(N / 128) + 1) (start / 128 + b) per head:
+// start / 128 + b grows by at least ceil(L / 128) from one sequence to the
+// next, so no prefix over the lengths (a launch of its own before) is needed.
 // Inside a tile (8 KiB): [wave w][key sub-tile kt][lane] 16-byte packs, the
 // A operand of dK/dV's dK MFMA: keys 32 w + 16 kt + li, queries
 // {4g .. 4g+3, 16+4g .. 16+4g+3} of the tile (times the query's e4m3 scale).
@@ -334,7 +355,8 @@ __host__ __device__ inline int64_t ds_tiles(int64_t L) {
 }
 __device__ __forceinline__ uint8_t* ds_tile(const AttnParams& p, const SeqCtx& c, int kb, int qt) {
   const int64_t QT = (c.L + 31) / 32;
-  const int64_t idx = p.ds_base[c.b] * p.H + (int64_t)c.h * ds_tiles(c.L) + (int64_t)kb * QT -
+  const int64_t base = 2 * ((int64_t)(p.N + 127) / 128 + 1) * (c.start / 128 + c.b);
+  const int64_t idx = base * p.H + (int64_t)c.h * ds_tiles(c.L) + (int64_t)kb * QT -
                       2 * (int64_t)kb * kb - 2 * (int64_t)kb + qt;
   return p.ds_ws + idx * kDsTileBytes;
 }
@@ -402,6 +424,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
 
   SeqCtx sc;
   if (!seq_ctx(p, /*heavy_last=*/true, sc)) return;
+  if (sc.tail > 0) zero_tail<D>(sc, p.N, p.out, p.o_rs);
   const int L = sc.L, h = sc.h;
   const int m0 = sc.blk * C::BM;
   if (m0 >= L) return;
@@ -758,6 +781,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_pv8_kernel(AttnParams p)
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   SeqCtx sc;
   if (!seq_ctx(p, /*heavy_last=*/true, sc)) return;
+  if (sc.tail > 0) zero_tail<128>(sc, p.N, p.out, p.o_rs);
   const int L = sc.L, h = sc.h;
   const int m0 = sc.blk * C::BM;
   if (m0 >= L) return;
@@ -1323,6 +1347,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
 
   SeqCtx sc;
   if (!seq_ctx(p, /*heavy_last=*/true, sc)) return;
+  if (sc.tail > 0) zero_tail<D>(sc, p.N, p.dq, p.dq_rs);
   const int L = sc.L, h = sc.h;
   const int m0 = sc.blk * C::BM;
   if (m0 >= L) return;
@@ -1588,6 +1613,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_ws_kernel(AttnParams 
 
   SeqCtx sc;
   if (!seq_ctx(p, /*heavy_last=*/true, sc)) return;
+  if (sc.tail > 0) zero_tail<D>(sc, p.N, p.dq, p.dq_rs);
   const int L = sc.L, h = sc.h;
   const int m0 = sc.blk * C::BM;
   if (m0 >= L) return;
@@ -1858,6 +1884,10 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
 
   SeqCtx sc;
   if (!seq_ctx(p, /*heavy_last=*/false, sc)) return;
+  if (sc.tail > 0) {
+    zero_tail<D>(sc, p.N, p.dk, p.dk_rs);
+    zero_tail<D>(sc, p.N, p.dv, p.dv_rs);
+  }
   const int L = sc.L, h = sc.h;
   const int n0 = sc.blk * C::BN;
   if (n0 >= L) return;
@@ -2248,14 +2278,16 @@ struct F8Bwd {
 // with nq = ceil(L / 128) tiles, (sequence, head) items hold nq (nq + 1) / 2
 // tiles, kb-major.  Inside a tile: [wave w][half hf][lane][16 bytes], the
 // 4 dwords qs = 0..3 of lane (li, g) being keys 16 w + li, queries
-// 64 hf + 16 qs + 4 g + (0..3).
+// 64 hf + 16 qs + 4 g + (0..3).  A sequence's tiles start at the closed form
+// ceil((ceil(N / 128) + 1) (start / 128 + b) / 2) per head (as ds_tile's).
 __host__ __device__ inline int64_t f8_tiles(int64_t L) {
   const int64_t nq = (L + 127) / 128;
   return nq * (nq + 1) / 2;
 }
 __device__ __forceinline__ uint8_t* f8_tile(const AttnParams& p, const SeqCtx& c, int kb, int qt) {
   const int64_t nq = (c.L + 127) / 128;
-  const int64_t idx = p.ds_base[c.b] * p.H + (int64_t)c.h * f8_tiles(c.L) + (int64_t)kb * nq -
+  const int64_t base = (((int64_t)(p.N + 127) / 128 + 1) * (c.start / 128 + c.b) + 1) / 2;
+  const int64_t idx = base * p.H + (int64_t)c.h * f8_tiles(c.L) + (int64_t)kb * nq -
                       (int64_t)kb * (kb - 1) / 2 + (qt - kb);
   return p.ds_ws + idx * F8Bwd::TILE;
 }
@@ -2298,6 +2330,10 @@ __global__ void __launch_bounds__(F8Bwd::NT, 3) hstu_bwd_f8_dkdv_kernel(AttnPara
   SeqCtx sc;
   int half = 0;
   if (!seq_ctx(p, /*heavy_last=*/false, sc, &half)) return;
+  if (sc.tail > 0 && half == 0) {
+    zero_tail<128>(sc, p.N, p.dk, p.dk_rs);
+    zero_tail<128>(sc, p.N, p.dv, p.dv_rs);
+  }
   const int L = sc.L, h = sc.h;
   const int n0 = sc.blk * C::BN;
   if (n0 >= L) return;
@@ -2553,6 +2589,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_f8_dq_kernel(AttnParams 
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   SeqCtx sc;
   if (!seq_ctx(p, /*heavy_last=*/true, sc)) return;
+  if (sc.tail > 0) zero_tail<128>(sc, p.N, p.dq, p.dq_rs);
   const int L = sc.L, h = sc.h;
   const int qt = sc.blk;
   const int m0 = qt * C::BM;
@@ -2822,13 +2859,10 @@ __device__ __forceinline__ int64_t dq_blocks(const int64_t* seq_offsets, int b, 
   return (min(seq_offsets[b + 1] - seq_offsets[b], (int64_t)N) + 127) / 128;
 }
 
-// base[b] = sum over sequences b' < b of f8_tiles(min(length, N)); base[B] =
-// the total; dq_base the same prefix of 128-query blocks (the bias-gradient
-// rows).
-__device__ void f8_tile_prefix(const int64_t* seq_offsets, int B, int N, int64_t* base, int64_t* dq_base) {
+// dq_base[b] = 128-query blocks of the sequences before b, dq_base[B] the
+// total (the bias-gradient rows), by one 1024-thread block.
+__device__ void dq_block_prefix(const int64_t* seq_offsets, int B, int N, int64_t* dq_base) {
   __shared__ int64_t part[1024];
-  seq_exclusive_scan(B, [&](int b) { return f8_tiles(min(seq_offsets[b + 1] - seq_offsets[b], (int64_t)N)); },
-                     part, base);
   seq_exclusive_scan(B, [&](int b) { return dq_blocks(seq_offsets, b, N); }, part, dq_base);
 }
 
@@ -2993,6 +3027,21 @@ __device__ void schedule_block(const int64_t* seq_offsets, int B, int H, int N, 
   }
 }
 
+// A direct grid (no schedule) for up to 1280 blocks, 2.5 rounds of the chip's
+// 512 workgroup slots: the call's set-up launch (5 us and its gap) goes.
+// Beyond, the schedule's balance and L2 reuse are worth it.  Measured (us,
+// schedule / direct; bf16 forward, backward; H = 4): 8 sequences of up to 1024
+// (256 blocks) 34.8 / 29.2, 78.1 / 69.4; 32 (1024) 38.6 / 35.6, 91.8 / 90.6;
+// 100 of up to 300 (1200) 28.1 / 24.4, 56.9 / 50.0; 64 of up to 1024 (2048)
+// 59.1 / 61.0, 157.7 / 165.8; 128 (4096) 119.5 / 136.2, 317 / 368.
+// A call whose set-up launch stays for other work (`prep`: a bias in the
+// backward, the full-FP8 backward's scale maxima) takes it only where the
+// schedule's whole items would leave XCDs idle or uneven: fewer than 16 items.
+// Full-FP8 backward: 2 items of up to 6 000 186.7 / 169.9, 4 of 3 001
+// 104.1 / 99.0; 128 items of up to 1024 81.1 / 85.2.
+bool direct_grid(int B, int H, int N, bool prep) {
+  return (int64_t)B * H * ((N + 127) / 128) <= 1280 && (!prep || B * H < 16);
+}
 // Point p at the block schedule in ws (sched_ints(B, H) ints).
 void use_schedule(AttnParams& p, int B, int H, int* ws) {
   p.sched_cap = sched_cap(B, H);
@@ -3000,8 +3049,12 @@ void use_schedule(AttnParams& p, int B, int H, int* ws) {
   p.sched_start = ws + 8 * p.sched_cap;
   p.sched_count = p.sched_start + 8 * (p.sched_cap + 1);
 }
-// grid covering every XCD's longest possible list
-int sched_grid(int B, int H, int N) { return 8 * sched_cap(B, H) * ((N + 127) / 128); }
+// workgroups (pairs, for the full-FP8 dK/dV): every XCD's longest possible
+// list, or every block of a direct grid, a multiple of 8
+int sched_grid(int B, int H, int N, bool direct) {
+  const int nb = (N + 127) / 128;
+  return direct ? (B * H * nb + 7) / 8 * 8 : 8 * sched_cap(B, H) * nb;
+}
 
 int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 int64_t bias_ext_bytes(int H, int N) { return align256((int64_t)H * bias_ext_len(N) * 4); }
@@ -3015,12 +3068,12 @@ int64_t sched_bytes(int B, int H) { return align256(sched_ints(B, H) * 4); }
 // Forward workspace: the block schedule.
 int64_t fwd_workspace_bytes(int B, int H) { return sched_bytes(B, H); }
 // Backward workspace: [block schedule][pre-clamped bias rows][bf16 copy of
-// e4m3 q][bias-gradient rows][their chunk sums][dQ block prefix][dS tile
-// prefix][dS tiles]; byte offsets of each part.  The dS tiles are sized by a bound that needs no lengths:
+// e4m3 q][bias-gradient rows][their chunk sums][dQ block prefix][dS
+// tiles]; byte offsets of each part.  The dS tiles are sized by a bound that needs no lengths:
 // ds_tiles(L) <= 2 nb (nb + 1) with nb = ceil(L / 128) <= ceil(N / 128), so
 // the sum over sequences is at most 2 (ceil(N/128) + 1) (ceil(T/128) + B).
 struct BwdWs {
-  int64_t sched, bias_ext, q16, part, chunks, dq_base, ds_base, ds, total;
+  int64_t sched, bias_ext, q16, part, chunks, dq_base, ds, total;
 };
 int64_t ds_tiles_bound(int64_t T, int B, int N) { return 2 * ((N + 127) / 128 + 1) * ((T + 127) / 128 + B); }
 BwdWs bwd_ws(int dtype, int64_t T, int B, int H, int D, int N, int R) {
@@ -3038,30 +3091,12 @@ BwdWs bwd_ws(int dtype, int64_t T, int B, int H, int D, int N, int R) {
   if (R > 0) o += dbias_chunks_bytes(H, R);
   w.dq_base = o;
   o += align256(((int64_t)B + 1) * 8);
-  w.ds_base = o;
-  o += align256(((int64_t)B + 1) * 8);
   w.ds = o;
   o += ds_tiles_bound(T, B, N) * H * kDsTileBytes;
   w.total = o;
   return w;
 }
 
-
-// base[b] = sum over sequences b' < b of ds_tiles(min(length, N)); base[B] =
-// the total; dq_base (if not null) the same prefix of 128-query blocks.
-__global__ void __launch_bounds__(1024) ds_tile_prefix(const int64_t* seq_offsets, int B, int N, int64_t* base,
-                                                       int64_t* dq_base) {
-  __shared__ int64_t part[1024];
-  seq_exclusive_scan(B, [&](int b) { return ds_tiles(min(seq_offsets[b + 1] - seq_offsets[b], (int64_t)N)); },
-                     part, base);
-  if (dq_base != nullptr) seq_exclusive_scan(B, [&](int b) { return dq_blocks(seq_offsets, b, N); }, part, dq_base);
-}
-
-// dq_base alone (the recomputing dQ kernel's bias-gradient rows).
-__global__ void __launch_bounds__(1024) dq_block_prefix(const int64_t* seq_offsets, int B, int N, int64_t* dq_base) {
-  __shared__ int64_t part[1024];
-  seq_exclusive_scan(B, [&](int b) { return dq_blocks(seq_offsets, b, N); }, part, dq_base);
-}
 
 // Chunk c of head h's bias-gradient rows: the sum of rows c * per ..
 // min((c + 1) * per, n) - 1 in a fixed order, n = dq_base[B] rows per head.
@@ -3133,33 +3168,33 @@ __device__ void zero_rows_beyond_n(const int64_t* seq_offsets, int N, int width,
 
 // The small set-up work of an attention call in one launch of 1024-thread
 // blocks, by block role (each block takes one role, so every barrier inside
-// a role is block-uniform): the block schedule (one block, if sched); the FP8
-// backward's tile and dQ-block prefixes (one block) and the partial maxima of
-// its q and k scales (kScaleParts blocks), if tile_base; the pre-clamped bias rows (bias_bx blocks per head,
-// if bias_ext); rows past N zeroed in up to three outputs (kPrepZero blocks
-// per sequence, if z[0]).  The roles touch disjoint memory.
+// a role is block-uniform): the block schedule (one block, if sched); the
+// dQ-block prefix (one block, if dq_base); the partial maxima of the FP8
+// backward's q and k scales (kScaleParts blocks, if f8max); the pre-clamped
+// bias rows (bias_bx blocks per head, if bias_ext); rows past N zeroed in up
+// to three outputs (kPrepZero blocks per sequence, if z[0]).  The roles touch
+// disjoint memory; a call without any launches nothing.
 constexpr int kPrepZero = 4;
 struct PrepArgs {
   const int64_t* seq_offsets;
   int B, H, N;
-  int* sched;  // null: no schedule block
-  int64_t* tile_base;
+  int* sched;
   int64_t* dq_base;
-  unsigned* f8max;  // tile_base null: no prefix and no scale blocks
+  unsigned* f8max;
   const float* qs;
   const float* ks;
   int64_t ntok;
   int sH;
   int64_t srs, shs;
   const float* bias;
-  float* bias_ext;  // null: no bias blocks
+  float* bias_ext;
   int R, bias_bx;
   int width;
-  uint16_t* z[3];  // z[0] null: no zeroing blocks
+  uint16_t* z[3];
   int64_t zrs[3];
 };
 int prep_blocks(const PrepArgs& a) {
-  return (a.sched ? 1 : 0) + (a.tile_base ? 1 + kScaleParts : 0) + (a.bias_ext ? a.H * a.bias_bx : 0) +
+  return (a.sched ? 1 : 0) + (a.dq_base ? 1 : 0) + (a.f8max ? kScaleParts : 0) + (a.bias_ext ? a.H * a.bias_bx : 0) +
          (a.z[0] ? kPrepZero * a.B : 0);
 }
 __global__ void __launch_bounds__(1024) attn_prep(PrepArgs a) {
@@ -3171,16 +3206,19 @@ __global__ void __launch_bounds__(1024) attn_prep(PrepArgs a) {
     }
     blk -= 1;
   }
-  if (a.tile_base) {
+  if (a.dq_base) {
     if (blk == 0) {
-      f8_tile_prefix(a.seq_offsets, a.B, a.N, a.tile_base, a.dq_base);
+      dq_block_prefix(a.seq_offsets, a.B, a.N, a.dq_base);
       return;
     }
-    if (blk <= kScaleParts) {
-      f8_scale_part(a.qs, a.ks, a.ntok, a.sH, a.srs, a.shs, a.f8max, blk - 1);
+    blk -= 1;
+  }
+  if (a.f8max) {
+    if (blk < kScaleParts) {
+      f8_scale_part(a.qs, a.ks, a.ntok, a.sH, a.srs, a.shs, a.f8max, blk);
       return;
     }
-    blk -= 1 + kScaleParts;
+    blk -= kScaleParts;
   }
   if (a.bias_ext) {
     const int nb = a.H * a.bias_bx;
@@ -3308,18 +3346,22 @@ int fwd_launch(int dtype, const void* q, const void* k, const void* v, int64_t q
   p.contextual_seq_len = contextual_seq_len;
   const bool generic = num_targets != nullptr || max_attn_len > 0 || contextual_seq_len > 0;
   p.blocks_per_seq = (max_seq_len + 127) / 128;
-  const int grid = sched_grid(B, H, max_seq_len);
+  const bool direct = direct_grid(B, H, max_seq_len, /*prep=*/false);
+  const int grid = sched_grid(B, H, max_seq_len, direct);
   p.bias = attn_bias;
   p.bias_R = bias_R;
   // the block schedule, and the rows past max_seq_len zeroed, in one launch
+  // (a direct grid has no schedule and zeroes them itself: nothing to launch)
   PrepArgs pa = prep_args(seq_offsets, B, H, max_seq_len);
-  pa.sched = sched_ws;
-  pa.width = H * D;
-  pa.z[0] = p.out;
-  pa.zrs[0] = p.o_rs;
+  if (!direct) {
+    pa.sched = sched_ws;
+    pa.width = H * D;
+    pa.z[0] = p.out;
+    pa.zrs[0] = p.o_rs;
+  }
   hipError_t e = launch_prep(pa, stream);
   if (e != hipSuccess) return (int)e;
-  use_schedule(p, B, H, sched_ws);
+  if (!direct) use_schedule(p, B, H, sched_ws);
 #define HSTU_FWD(DD, F8, G, BB) launch(hstu_fwd_kernel<DD, F8, G, BB>, FwdCfg<DD, F8>::LDS, grid, p, stream)
 #define HSTU_FWD_B(DD, F8, G) (has_bias ? HSTU_FWD(DD, F8, G, true) : HSTU_FWD(DD, F8, G, false))
   const bool has_bias = attn_bias != nullptr;
@@ -3507,11 +3549,12 @@ int attn_bwd_impl(int parts, int dtype, const void* dout, int64_t dout_row_strid
   p.contextual_seq_len = contextual_seq_len;
   p.blocks_per_seq = (max_seq_len + 127) / 128;
   const bool generic = num_targets != nullptr || max_attn_len > 0 || contextual_seq_len > 0;
-  const int grid = sched_grid(B, H, max_seq_len);
+  const bool has_bias = attn_bias != nullptr;
+  const bool direct = direct_grid(B, H, max_seq_len, has_bias);
+  const int grid = sched_grid(B, H, max_seq_len, direct);
   p.bias = attn_bias;
   p.bias_R = bias_R;
   p.dbias = dbias;
-  const bool has_bias = attn_bias != nullptr;
   hipError_t e;
   const BwdWs wl = bwd_ws(dtype, total_tokens, B, H, D, max_seq_len, has_bias ? bias_R : 0);
   if (total_tokens < 0 || workspace_bytes < wl.total || workspace == nullptr) return HSTU_E_BAD_ARG;
@@ -3522,32 +3565,33 @@ int attn_bwd_impl(int parts, int dtype, const void* dout, int64_t dout_row_strid
     if (lds > kMaxLdsBytes) return HSTU_E_UNSUPPORTED;
   }
   uint8_t* ws = (uint8_t*)workspace;
-  // the block schedule, the pre-clamped bias rows (dK/dV) and the rows past
-  // max_seq_len of this half's outputs zeroed, in one launch
+  // the block schedule, the pre-clamped bias rows (dK/dV), the dQ-block prefix
+  // (dQ with a bias) and the rows past max_seq_len of this half's outputs
+  // zeroed, in one launch; a direct grid needs the middle two only
   PrepArgs pa = prep_args(seq_offsets, B, H, max_seq_len);
-  pa.sched = (int*)(ws + wl.sched);
+  if (!direct) pa.sched = (int*)(ws + wl.sched);
+  if ((parts & kBwdDq) && has_bias) pa.dq_base = (int64_t*)(ws + wl.dq_base);
   if ((parts & kBwdDkdv) && has_bias) {
     pa.bias = attn_bias;
     pa.R = bias_R;
     pa.bias_ext = (float*)(ws + wl.bias_ext);
     pa.bias_bx = (bias_ext_len(max_seq_len) + 1023) / 1024;
   }
-  pa.width = H * D;
-  pa.z[0] = (parts & kBwdDq) ? p.dq : p.dk;
-  pa.zrs[0] = (parts & kBwdDq) ? p.dq_rs : p.dk_rs;
-  pa.z[1] = (parts & kBwdDkdv) ? p.dk : (uint16_t*)nullptr;
-  pa.zrs[1] = p.dk_rs;
-  pa.z[2] = (parts & kBwdDkdv) ? p.dv : (uint16_t*)nullptr;
-  pa.zrs[2] = p.dv_rs;
+  if (!direct) {
+    pa.width = H * D;
+    pa.z[0] = (parts & kBwdDq) ? p.dq : p.dk;
+    pa.zrs[0] = (parts & kBwdDq) ? p.dq_rs : p.dk_rs;
+    pa.z[1] = (parts & kBwdDkdv) ? p.dk : (uint16_t*)nullptr;
+    pa.zrs[1] = p.dk_rs;
+    pa.z[2] = (parts & kBwdDkdv) ? p.dv : (uint16_t*)nullptr;
+    pa.zrs[2] = p.dv_rs;
+  }
   e = launch_prep(pa, stream);
   if (e != hipSuccess) return (int)e;
-  use_schedule(p, B, H, (int*)(ws + wl.sched));
+  if (!direct) use_schedule(p, B, H, (int*)(ws + wl.sched));
   if (!generic) {
     // dS tiles pass from the dK/dV kernel to the dQ kernel through the workspace
-    p.ds_base = (const int64_t*)(ws + wl.ds_base);
     p.ds_ws = ws + wl.ds;
-    hipLaunchKernelGGL(ds_tile_prefix, dim3(1), dim3(1024), 0, stream, seq_offsets, B, max_seq_len,
-                       (int64_t*)(ws + wl.ds_base), has_bias ? (int64_t*)(ws + wl.dq_base) : (int64_t*)nullptr);
   }
   if (parts & kBwdDkdv) {
     if (has_bias) p.bias_ext = (const float*)(ws + wl.bias_ext);
@@ -3577,9 +3621,6 @@ int attn_bwd_impl(int parts, int dtype, const void* dout, int64_t dout_row_strid
       p.dbias_part = (float*)(ws + wl.part);
       p.dq_base = (const int64_t*)(ws + wl.dq_base);
       p.dbias_w = generic ? 2 * bias_R - 1 : bias_R;
-      if (generic)
-        hipLaunchKernelGGL(dq_block_prefix, dim3(1), dim3(1024), 0, stream, seq_offsets, B, max_seq_len,
-                           (int64_t*)(ws + wl.dq_base));
     }
     // dQ (+ bias gradient): 128-query blocks, longest key range first.  With
     // the causal mask, from the dS tiles the dK/dV kernel stored.
@@ -3655,7 +3696,7 @@ namespace {
 // bound that needs no lengths: sum_b nq_b (nq_b + 1) / 2 <= (nq_max + 1) / 2 *
 // (ceil(T / 128) + B), nq_max = ceil(N / 128).
 struct F8Ws {
-  int64_t sched, bias_ext, part, chunks, dq_base, maxv, base, tiles, total;
+  int64_t sched, bias_ext, part, chunks, dq_base, maxv, tiles, total;
 };
 int64_t f8_tiles_bound(int64_t T, int B, int N) {
   const int64_t nq = (N + 127) / 128;
@@ -3676,8 +3717,6 @@ F8Ws f8_ws(int64_t T, int B, int H, int N, int R) {
   o += align256(((int64_t)B + 1) * 8);
   w.maxv = o;
   o += align256(kScaleParts * 2 * 4);
-  w.base = o;
-  o += align256(((int64_t)B + 1) * 8);
   w.tiles = o;
   o += f8_tiles_bound(T, B, N) * H * F8Bwd::TILE;
   w.total = o;
@@ -3769,19 +3808,18 @@ int attn_bwd_fp8_impl(int parts, const void* dout8, const void* dout_e8, int64_t
   p.p8_scale = ldexpf(1.0f, p8_scale_log2);
   p.ds8_scale = ldexpf(1.0f, ds8_scale_log2);
   p.f8max = (const unsigned*)(ws + wl.maxv);
-  p.ds_base = (const int64_t*)(ws + wl.base);
   p.ds_ws = ws + wl.tiles;
-  const int grid = sched_grid(B, H, max_seq_len);
+  const bool direct = direct_grid(B, H, max_seq_len, /*prep=*/true);
+  const int grid = sched_grid(B, H, max_seq_len, direct);
   // One launch for the set-up: with the dK/dV half, the block schedule, the
-  // tile and dQ-block prefixes (and the scale-maximum reset) and the
-  // pre-clamped bias rows, all read by both halves (the dQ half, which runs
-  // after it on the same workspace, builds none of them); and the rows past
-  // max_seq_len of this half's outputs zeroed.
+  // dQ-block prefix, the scale maxima and the pre-clamped bias rows, all read by
+  // both halves (the dQ half, which runs after it on the same workspace, builds
+  // none of them); and the rows past max_seq_len of this half's outputs
+  // zeroed.  A direct grid has no schedule and zeroes those rows itself.
   PrepArgs pa = prep_args(seq_offsets, B, H, max_seq_len);
   if (parts & kBwdDkdv) {
-    pa.sched = (int*)(ws + wl.sched);
-    pa.tile_base = (int64_t*)(ws + wl.base);
-    pa.dq_base = (int64_t*)(ws + wl.dq_base);
+    if (!direct) pa.sched = (int*)(ws + wl.sched);
+    if (has_bias) pa.dq_base = (int64_t*)(ws + wl.dq_base);
     pa.f8max = (unsigned*)(ws + wl.maxv);
     const bool per_token = scale_row_stride || scale_head_stride;
     pa.qs = q_scale;
@@ -3797,16 +3835,18 @@ int attn_bwd_fp8_impl(int parts, const void* dout8, const void* dout_e8, int64_t
       pa.bias_bx = (bias_ext_len(max_seq_len) + 1023) / 1024;
     }
   }
-  pa.width = H * D;
-  pa.z[0] = (parts & kBwdDq) ? p.dq : p.dk;
-  pa.zrs[0] = (parts & kBwdDq) ? p.dq_rs : p.dk_rs;
-  pa.z[1] = (parts & kBwdDkdv) ? p.dk : (uint16_t*)nullptr;
-  pa.zrs[1] = p.dk_rs;
-  pa.z[2] = (parts & kBwdDkdv) ? p.dv : (uint16_t*)nullptr;
-  pa.zrs[2] = p.dv_rs;
+  if (!direct) {
+    pa.width = H * D;
+    pa.z[0] = (parts & kBwdDq) ? p.dq : p.dk;
+    pa.zrs[0] = (parts & kBwdDq) ? p.dq_rs : p.dk_rs;
+    pa.z[1] = (parts & kBwdDkdv) ? p.dk : (uint16_t*)nullptr;
+    pa.zrs[1] = p.dk_rs;
+    pa.z[2] = (parts & kBwdDkdv) ? p.dv : (uint16_t*)nullptr;
+    pa.zrs[2] = p.dv_rs;
+  }
   hipError_t e = launch_prep(pa, stream);
   if (e != hipSuccess) return (int)e;
-  use_schedule(p, B, H, (int*)(ws + wl.sched));
+  if (!direct) use_schedule(p, B, H, (int*)(ws + wl.sched));
   if (parts & kBwdDkdv) {
     const bool per_token = scale_row_stride || scale_head_stride;
     if (has_bias) p.bias_ext = (const float*)(ws + wl.bias_ext);

@@ -649,3 +649,40 @@ def test_full_fp8_backward_rows_past_max_seq_len(hip_lib):
         assert torch.equal(a[~keep], torch.zeros_like(a[~keep])), f"{name}: rows past N not zero"
         assert torch.equal(a[keep], b), f"{name}: kept rows differ from the cut batch"
     assert orc.rel_l2(dbc.double(), db.double()) <= 1e-6  # the same pairs, summed in another block order
+
+
+@pytest.mark.parametrize("kind,D,H", [("bf16", 64, 1), ("bf16", 128, 4), ("targets", 128, 2), ("bias", 128, 2),
+                                      ("e4m3", 128, 1), ("e4m3", 128, 4)])
+def test_direct_grid_same_bytes(hip_lib, kind, D, H):
+    """A few sequences (direct grid: no schedule, rows past N zeroed by the
+    attention kernels) give the bytes of the same sequences among enough empty
+    ones for the scheduled grid; lengths around 128 and past N."""
+    ops = _ops()
+    N, lengths = 300, [300, 0, 129, 411, 1, 128, 300 + 257]
+    many = lengths + [0] * 1300
+    q, k, v, offs = _case(lengths, H, D, seed=D + H)
+    T = q.shape[0]
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(DEV)
+    q, k, v = (t.to(DEV) for t in (q, k, v))
+    scales = [None] * 3
+    if kind == "e4m3":
+        q, k, v = ((t.float() * 100).to(torch.float8_e4m3fn) for t in (q, k, v))
+        g = torch.Generator(device=DEV).manual_seed(3)
+        scales = [0.005 + 0.01 * torch.rand(T, H, device=DEV, generator=g) for _ in range(3)]
+    bias = orc.make_bias(H, 64, seed=2, std=0.3).to(DEV) if kind == "bias" else None
+    res = []
+    for lens in (lengths, many):
+        off = orc.offsets_from_lengths(lens).to(DEV)
+        nt = torch.tensor([2, 0, 1, 3, 1, 1, 9] + [0] * (len(lens) - 7), device=DEV) if kind == "targets" else None
+        out = ops.triton_hstu_attention_fwd(N, 0.1, q, k, v, off, nt, 0, 0, None, False, 0, *scales, attn_bias=bias,
+                                            fp8_pv=kind == "e4m3")
+        grads = [torch.full(q.shape, float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(3)]
+        db = None if bias is None else torch.empty_like(bias)
+        ops.triton_hstu_attention_bwd(dout, q, k, v, *grads, off, nt, N, 0.1, 0, 0, None, False, 0, *scales,
+                                      attn_bias=bias, dbias=db, full_fp8=kind == "e4m3")
+        res.append([out, *grads])
+    torch.cuda.synchronize()
+    pos = torch.cat([torch.arange(n) for n in lengths])
+    for name, a, b in zip(("out", "dq", "dk", "dv"), *res):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16)), name
+        assert bool((a.cpu()[pos >= N] == 0).all()) and not bool(torch.isnan(a).any()), name
