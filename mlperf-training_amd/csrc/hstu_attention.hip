@@ -299,6 +299,8 @@ struct SeqCtx {
 //  * direct (no schedule): block m of item u % (B H), m = u / (B H), u the
 //    workgroup (pair), so all items' heaviest blocks come first and one item's
 //    blocks spread over the XCDs when there are few items.
+// ROWS: rows of a block; 64 only with a direct grid.
+template <int ROWS = 128>
 __device__ __forceinline__ bool seq_ctx(const AttnParams& p, bool heavy_last, SeqCtx& c, int* half = nullptr) {
   const int x = blockIdx.x & 7, k = half ? blockIdx.x >> 4 : blockIdx.x >> 3;
   if (half) *half = (blockIdx.x >> 3) & 1;
@@ -325,7 +327,7 @@ __device__ __forceinline__ bool seq_ctx(const AttnParams& p, bool heavy_last, Se
   c.start = p.seq_offsets[c.b];
   const int64_t len = p.seq_offsets[c.b + 1] - c.start;
   c.L = min((int)len, p.N);
-  const int nb = (c.L + 127) / 128;
+  const int nb = (c.L + ROWS - 1) / ROWS;
   c.blk = heavy_last ? nb - 1 - m : m;
   c.tail = p.sched_items == nullptr && m == 0 ? (int)len - c.L : 0;
   return m < nb;
@@ -382,9 +384,10 @@ __device__ __forceinline__ void wait_vm_le() {
 // r -> r + 16.
 __host__ __device__ constexpr int swz128(int r) { return ((r >> 1) & 7) ^ (((r >> 5) & 1) << 2); }
 
-template <int D, bool FP8>
+// QT: 16-query sub-tiles per wave
+template <int D, bool FP8, int QT = 2>
 struct FwdCfg {
-  static constexpr int BM = 128, BN = 64, KT = BN / 16, DT = D / 16, KS = D / 32;
+  static constexpr int BM = 64 * QT, BN = 64, KT = BN / 16, DT = D / 16, KS = D / 32;
   static constexpr int ES = FP8 ? 1 : 2;
   // bf16 rows at a pitch of row bytes + 32 (== 32 mod 64) for the 16-row
   // ds_read_b128 operand reads and the ds_read_b64_tr_b16 V reads; the e4m3
@@ -416,14 +419,18 @@ struct FwdStage {
   float bias;  // threads 0..BM+BN-2: one bias value of the tile's offset band
 };
 
-template <int D, bool FP8, bool GENERIC, bool BIAS>
+// QT = 1: blocks of 64 queries, for grids that leave the chip idle.  The time
+// is then the longest block's serial tiles, and with half the queries a tile
+// costs a wave half the MFMAs and SiLU; every element is the same sum in the
+// same order.
+template <int D, bool FP8, bool GENERIC, bool BIAS, int QT = 2>
 __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
-  using C = FwdCfg<D, FP8>;
+  using C = FwdCfg<D, FP8, QT>;
   static_assert(!FP8 || D == 128, "e4m3 path is specialised for D = 128");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
   SeqCtx sc;
-  if (!seq_ctx(p, /*heavy_last=*/true, sc)) return;
+  if (!seq_ctx<C::BM>(p, /*heavy_last=*/true, sc)) return;
   if (sc.tail > 0) zero_tail<D>(sc, p.N, p.out, p.o_rs);
   const int L = sc.L, h = sc.h;
   const int m0 = sc.blk * C::BM;
@@ -432,7 +439,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15,
             g = lane >> 4;
-  const int mw0 = m0 + wave * 32;
+  const int mw0 = m0 + wave * 16 * QT;
   const bool wave_active = mw0 < L;
 
   const uint32_t krs = (uint32_t)(p.k_rs * C::ES), vrs = (uint32_t)(p.v_rs * C::ES);
@@ -466,11 +473,11 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
   }
 
   // Q fragments (B operand of S^T = K.Q^T): lane holds query mw0+16qt+li.
-  u32x4 qf[2][C::KS];
-  i32x8 qf8[2];
-  float cq[2];
+  u32x4 qf[QT][C::KS];
+  i32x8 qf8[QT];
+  float cq[QT];
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
     const int row = mw0 + qt * 16 + li;
     const bool ok = row < L;
     const uint8_t* src = qb + (int64_t)row * qrs;
@@ -494,9 +501,9 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
     }
   }
 
-  f32x4 o[2][C::DT];
+  f32x4 o[QT][C::DT];
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt)
+  for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt) o[qt][dt] = zero4();
 
@@ -509,8 +516,12 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
   }
   const int ntiles = (n_end + C::BN - 1) / C::BN;
 
-  FwdStage<D, FP8> stg;
-  auto load = [&](int n0) {
+  // tiles in registers on their way to LDS: one, or with QT = 1 two, so that a
+  // tile's loads have two tiles' time (a lone workgroup's tile is shorter than
+  // a memory round trip)
+  constexpr int NST = QT == 1 ? 2 : 1;
+  FwdStage<D, FP8> stages[NST];
+  auto load = [&](int n0, FwdStage<D, FP8>& stg) {
 #pragma unroll
     for (int i = 0; i < C::K_N; ++i) stg.k[i] = buf_ld128(krsrc, k_voff[i], n0 * krs);
 #pragma unroll
@@ -535,7 +546,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
       }
     }
   };
-  auto store = [&](uint8_t* buf) {
+  auto store = [&](uint8_t* buf, const FwdStage<D, FP8>& stg) {
 #pragma unroll
     for (int i = 0; i < C::K_N; ++i) *(u32x4*)(buf + k_loff[i]) = stg.k[i];
 #pragma unroll
@@ -576,45 +587,49 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
   // tr16: lane j of group g addresses row 4g + j/4 (+16 for the second half), column 4*(j%4)
   const int v_rd = C::V_OFF + (4 * g + (li >> 2)) * C::VP + (li & 3) * 8;
   // bias index of element (qt, kt, r) = bias_rd + 16*(qt-kt) - r
-  const int bias_rd = 32 * wave + (C::BN - 1) + li - 4 * g;
+  const int bias_rd = 16 * QT * wave + (C::BN - 1) + li - 4 * g;
 
   // positions of the lane's queries (generic masks)
-  int qid[2] = {0, 0};
+  int qid[QT] = {};
   if constexpr (GENERIC) {
-    qid[0] = mask_id(mw0 + li, mc);
-    qid[1] = mask_id(mw0 + 16 + li, mc);
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) qid[qt] = mask_id(mw0 + 16 * qt + li, mc);
   }
 
-  load(t_begin * C::BN);
-  store(smem + (t_begin & 1) * C::BUF);
+  load(t_begin * C::BN, stages[0]);
+  if (NST == 2 && t_begin + 1 < ntiles) load((t_begin + 1) * C::BN, stages[NST - 1]);
+  store(smem + (t_begin & 1) * C::BUF, stages[0]);
   __syncthreads();
 
-  for (int t = t_begin; t < ntiles; ++t) {
+  // one tile; PAR = (t - t_begin) % NST: tile t + NST goes to the stage that
+  // tile t left, tile t + 1's stage is stored at the end
+  auto tile = [&](int t, auto par_c) {
+    constexpr int PAR = decltype(par_c)::value;
     const int n0 = t * C::BN;
     const uint8_t* buf = smem + (t & 1) * C::BUF;
-    if (t + 1 < ntiles) load(n0 + C::BN);
+    if (t + NST < ntiles) load(n0 + NST * C::BN, stages[PAR]);
 
-    const MaskClass cls = GENERIC ? mask_class(mw0, mw0 + 31, n0, n0 + C::BN - 1, mc)
-                                  : n0 > mw0 + 31 ? kMaskNone : n0 + C::BN - 1 > mw0 ? kMaskSome : kMaskAll;
+    const MaskClass cls = GENERIC ? mask_class(mw0, mw0 + 16 * QT - 1, n0, n0 + C::BN - 1, mc)
+                                  : n0 > mw0 + 16 * QT - 1 ? kMaskNone : n0 + C::BN - 1 > mw0 ? kMaskSome : kMaskAll;
     if (wave_active && cls != kMaskNone) {
       // ---- S^T = K . Q^T : s[kt][qt], keys n0+16kt+4g+r, query mw0+16qt+li
-      f32x4 s[C::KT][2];
+      f32x4 s[C::KT][QT];
 #pragma unroll
       for (int kt = 0; kt < C::KT; ++kt) {
         const uint8_t* krow = buf + k_rd + kt * 16 * C::KP;
         if constexpr (FP8) {
           const uint8_t* kb = buf + kt * 16 * 128;
           i32x8 a = cat8(lds_ld128(kb + (kt < 2 ? ka0 : ka1)), lds_ld128(kb + (kt < 2 ? ka1 : ka0)));
-          s[kt][0] = mfma_fp8(a, qf8[0], zero4());
-          s[kt][1] = mfma_fp8(a, qf8[1], zero4());
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) s[kt][qt] = mfma_fp8(a, qf8[qt], zero4());
         } else {
-          s[kt][0] = zero4();
-          s[kt][1] = zero4();
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) s[kt][qt] = zero4();
 #pragma unroll
           for (int st = 0; st < C::KS; ++st) {
             u32x4 a = lds_ld128(krow + st * 64);
-            s[kt][0] = mfma_bf16(a, qf[0][st], s[kt][0]);
-            s[kt][1] = mfma_bf16(a, qf[1][st], s[kt][1]);
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt) s[kt][qt] = mfma_bf16(a, qf[qt][st], s[kt][qt]);
           }
         }
       }
@@ -623,7 +638,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
       // whole tile in the clamped bias region: one constant
       const bool bias_const = BIAS && (m0 - n0 - (C::BN - 1) >= R1);
       const float* bias_lds = (const float*)(buf + C::BIAS_OFF);
-      u32x4 pa[2][C::BN / 32];
+      u32x4 pa[QT][C::BN / 32];
       auto epilogue = [&](auto masked_tag, auto bconst_tag) {
         constexpr bool MASKED = decltype(masked_tag)::value;
         constexpr bool BCONST = decltype(bconst_tag)::value;
@@ -638,7 +653,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
             svv = f32x4{a[1], a[3], b[1], b[3]};
           }
 #pragma unroll
-          for (int qt = 0; qt < 2; ++qt) {
+          for (int qt = 0; qt < QT; ++qt) {
             float pv[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -678,21 +693,29 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
         for (int dt = 0; dt < C::DT; ++dt) {
           const uint8_t* vp = buf + v_rd + c * 32 * C::VP + dt * 32;
           u32x4 bv = cat_tr(lds_tr16(vp), lds_tr16(vp + 16 * C::VP));
-          o[0][dt] = mfma_bf16(pa[0][c], bv, o[0][dt]);
-          o[1][dt] = mfma_bf16(pa[1][c], bv, o[1][dt]);
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) o[qt][dt] = mfma_bf16(pa[qt][c], bv, o[qt][dt]);
         }
       }
       __builtin_amdgcn_s_setprio(0);
     }
 
-    if (t + 1 < ntiles) store(smem + ((t + 1) & 1) * C::BUF);
+    if (t + 1 < ntiles) store(smem + ((t + 1) & 1) * C::BUF, stages[(PAR + 1) % NST]);
     __syncthreads();
+  };
+  if constexpr (NST == 1) {
+    for (int t = t_begin; t < ntiles; ++t) tile(t, std::integral_constant<int, 0>{});
+  } else {
+    for (int t = t_begin; t < ntiles; t += 2) {
+      tile(t, std::integral_constant<int, 0>{});
+      if (t + 1 < ntiles) tile(t + 1, std::integral_constant<int, 1>{});
+    }
   }
 
   if (!wave_active) return;
   const float fin = -kLn2 * p.inv_n;
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = mw0 + qt * 16 + 4 * g + r;
@@ -3348,6 +3371,12 @@ int fwd_launch(int dtype, const void* q, const void* k, const void* v, int64_t q
   p.blocks_per_seq = (max_seq_len + 127) / 128;
   const bool direct = direct_grid(B, H, max_seq_len, /*prep=*/false);
   const int grid = sched_grid(B, H, max_seq_len, direct);
+  // 64-query blocks (bf16) while the 128-query ones are at most 512, one round
+  // of the chip.  Measured (us, 128 / 64; H = 4, D = 128): one sequence of 3 001
+  // (96 blocks) 71.0 / 50.8, D = 64 47.6 / 34.2; 16 of up to 1024 (512)
+  // 31.7 / 26.0; 8 of up to 2048 (512) 49.8 / 40.2; 32 of up to 1024 (1024)
+  // 38.2 / 41.2.
+  const bool half = direct && grid <= 512 && dtype == HSTU_DTYPE_BF16;
   p.bias = attn_bias;
   p.bias_R = bias_R;
   // the block schedule, and the rows past max_seq_len zeroed, in one launch
@@ -3375,6 +3404,15 @@ int fwd_launch(int dtype, const void* q, const void* k, const void* v, int64_t q
                  : launch(hstu_fwd_pv8_kernel<false>, Pv8Cfg::lds(max_seq_len), grid, p, stream);
   } else if (dtype == HSTU_DTYPE_FP8_E4M3) {
     e = generic ? HSTU_FWD_B(128, true, true) : HSTU_FWD_B(128, true, false);
+  } else if (half) {
+    const int grid64 = (B * H * ((max_seq_len + 63) / 64) + 7) / 8 * 8;
+#define HSTU_FWD64(DD, G, BB) \
+  launch(hstu_fwd_kernel<DD, false, G, BB, 1>, FwdCfg<DD, false, 1>::LDS, grid64, p, stream)
+#define HSTU_FWD64_B(DD, G) (has_bias ? HSTU_FWD64(DD, G, true) : HSTU_FWD64(DD, G, false))
+    if (D == 128) e = generic ? HSTU_FWD64_B(128, true) : HSTU_FWD64_B(128, false);
+    else e = generic ? HSTU_FWD64_B(64, true) : HSTU_FWD64_B(64, false);
+#undef HSTU_FWD64_B
+#undef HSTU_FWD64
   } else if (D == 128) {
     e = generic ? HSTU_FWD_B(128, false, true) : HSTU_FWD_B(128, false, false);
   } else {
