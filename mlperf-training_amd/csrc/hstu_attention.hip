@@ -2978,16 +2978,21 @@ inline int64_t sched_ints(int B, int H) {
   return 8 * cap + 8 * (cap + 1) + 8 + 2 * (int64_t)B;
 }
 
+// The time is its barriers and memory round trips, so the counts, ranks and
+// block counts stay in LDS for B and B H up to kSchedBins and 4 kSchedBins
+// (beyond: the scratch and the output), and the scans are wave scans.
 __device__ void schedule_block(const int64_t* seq_offsets, int B, int H, int N, int* ws) {
   const int cap = sched_cap(B, H);
   int* items = ws;
   int* start = items + 8 * cap;
   int* count = start + 8 * (cap + 1);
-  int* nbv = count + 8;
-  int* rank = nbv + B;
   __shared__ int bins[kSchedBins];
-  __shared__ int scan[kSchedBins];
-  const int tid = threadIdx.x;  // blockDim.x == kSchedBins
+  __shared__ int part[kSchedBins / 64];
+  __shared__ int nb_lds[kSchedBins], rank_lds[kSchedBins], cnt_lds[4 * kSchedBins];
+  int* nbv = B <= kSchedBins ? nb_lds : count + 8;
+  int* rank = B <= kSchedBins ? rank_lds : count + 8 + B;
+  int* cnt = 8 * (cap + 1) <= 4 * kSchedBins ? cnt_lds : start;  // block count of each XCD's j-th item
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;  // blockDim.x == kSchedBins
   bins[tid] = 0;
   __syncthreads();
   for (int b = tid; b < B; b += kSchedBins) {
@@ -2997,35 +3002,35 @@ __device__ void schedule_block(const int64_t* seq_offsets, int B, int H, int N, 
     atomicAdd(&bins[min(nb, kSchedBins - 1)], 1);
   }
   __syncthreads();
+  auto wave_scan = [&](int x) {  // inclusive
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o);
+      if (lane >= o) x += y;
+    }
+    return x;
+  };
   // exclusive prefix in descending bin order: first rank of bin v = sum of bins above v
   const int v = kSchedBins - 1 - tid;
-  const int mine = bins[v];
-  scan[tid] = mine;
+  const int mine = bins[v], incl = wave_scan(mine);
+  if (lane == 63) part[wave] = incl;
   __syncthreads();
-  for (int off = 1; off < kSchedBins; off <<= 1) {
-    const int add = tid >= off ? scan[tid - off] : 0;
-    __syncthreads();
-    scan[tid] += add;
-    __syncthreads();
-  }
-  bins[v] = scan[tid] - mine;
+  int before = 0;
+  for (int w = 0; w < wave; ++w) before += part[w];
+  bins[v] = before + incl - mine;
   __syncthreads();
   for (int b = tid; b < B; b += kSchedBins) rank[b] = atomicAdd(&bins[min(nbv[b], kSchedBins - 1)], 1);
   __syncthreads();
   // item r = rank*H + head -> XCD by snake order, dense index j on that XCD
-  for (int b = tid; b < B; b += kSchedBins) {
-    const int nb = nbv[b];
-    for (int h = 0; h < H; ++h) {
-      const int r = rank[b] * H + h, q = r & 15;
-      const int x = q < 8 ? q : 15 - q;
-      const int j = (r >> 4) * 2 + (q >= 8 ? 1 : 0);
-      items[x * cap + j] = b * H + h;
-      start[x * (cap + 1) + j] = nb;
-    }
+  for (int i = tid; i < B * H; i += kSchedBins) {
+    const int b = i / H, r = rank[b] * H + (i - b * H), q = r & 15;
+    const int x = q < 8 ? q : 15 - q;
+    const int j = (r >> 4) * 2 + (q >= 8 ? 1 : 0);
+    items[x * cap + j] = i;
+    cnt[x * (cap + 1) + j] = nbv[b];
   }
   __syncthreads();
   // per XCD (one wave each): exclusive scan of the block counts
-  const int wave = tid >> 6, lane = tid & 63;
   if (wave < 8) {
     const int x = wave, BH = B * H, full = BH >> 4, rem = BH & 15;
     const int n = 2 * full + (x < rem ? 1 : 0) + (15 - x < rem ? 1 : 0);
@@ -3033,15 +3038,10 @@ __device__ void schedule_block(const int64_t* seq_offsets, int B, int H, int N, 
     int carry = 0;
     for (int j0 = 0; j0 < n; j0 += 64) {
       const int j = j0 + lane;
-      const int c = j < n ? st[j] : 0;
-      int incl = c;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(incl, o);
-        if (lane >= o) incl += y;
-      }
-      if (j < n) st[j] = carry + incl - c;
-      carry += __shfl(incl, 63);
+      const int c = j < n ? cnt[x * (cap + 1) + j] : 0;
+      const int in = wave_scan(c);
+      if (j < n) st[j] = carry + in - c;
+      carry += __shfl(in, 63);
     }
     if (lane == 0) {
       st[n] = carry;
