@@ -332,6 +332,12 @@ __device__ __forceinline__ bool seq_ctx(const AttnParams& p, bool heavy_last, Se
   c.tail = p.sched_items == nullptr && m == 0 ? (int)len - c.L : 0;
   return m < nb;
 }
+// Query blocks come last (the most keys) to first; with a contextual prefix the
+// first block sees the whole sequence, so it goes before the others.
+template <int ROWS>
+__device__ __forceinline__ void prefix_block_first(const AttnParams& p, SeqCtx& c) {
+  if (p.contextual_seq_len > 0) c.blk = c.blk == (c.L + ROWS - 1) / ROWS - 1 ? 0 : c.blk + 1;
+}
 // Zeroes columns h D .. h D + D - 1 of rows N .. N + tail - 1 of a sequence's
 // output (the set-up launch does it when there is a schedule).
 template <int D>
@@ -366,6 +372,11 @@ __device__ __forceinline__ uint8_t* ds_tile(const AttnParams& p, const SeqCtx& c
 __device__ __forceinline__ MaskCtx mask_ctx(const AttnParams& p, const SeqCtx& c) {
   return mask_make(c.L, p.num_targets, c.b, p.max_attn_len, p.contextual_seq_len);
 }
+
+// Epilogue forms of a score tile: unmasked, the general mask, or its band form.
+using MaskNo = std::integral_constant<int, 0>;
+using MaskGen = std::integral_constant<int, 1>;
+using MaskBand = std::integral_constant<int, 2>;
 
 // =====================================================================
 // Forward.  Block = 128 query rows (32 per wave), key tiles of 64.
@@ -433,6 +444,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
   if (!seq_ctx<C::BM>(p, /*heavy_last=*/true, sc)) return;
   if (sc.tail > 0) zero_tail<D>(sc, p.N, p.out, p.o_rs);
   const int L = sc.L, h = sc.h;
+  if constexpr (GENERIC) prefix_block_first<C::BM>(p, sc);
   const int m0 = sc.blk * C::BM;
   if (m0 >= L) return;
   const MaskCtx mc = mask_ctx(p, sc);
@@ -640,7 +652,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
       const float* bias_lds = (const float*)(buf + C::BIAS_OFF);
       u32x4 pa[QT][C::BN / 32];
       auto epilogue = [&](auto masked_tag, auto bconst_tag) {
-        constexpr bool MASKED = decltype(masked_tag)::value;
+        constexpr int MASKED = decltype(masked_tag)::value;
         constexpr bool BCONST = decltype(bconst_tag)::value;
         const float bconst = (BIAS && BCONST) ? bias_lds[0] : 0.f;
 #pragma unroll
@@ -666,7 +678,9 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
               else val = t * sig_of_t(t);
               if constexpr (MASKED) {
                 const int i = mw0 + qt * 16 + li, j = n0 + kt * 16 + 4 * g + r;
-                const bool ok = GENERIC ? mask_pair(i, j, qid[qt], mask_id(j, mc), mc) : (j <= i);
+                const bool ok = !GENERIC            ? j <= i
+                                : MASKED == MaskGen() ? mask_pair(i, j, qid[qt], mask_id(j, mc), mc)
+                                                      : mask_band(i, j, mc);
                 val = ok ? val : 0.f;
               }
               pv[r] = val;
@@ -676,13 +690,13 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
           }
         }
       };
-      if (need_mask) {
-        if (bias_const) epilogue(std::true_type{}, std::true_type{});
-        else epilogue(std::true_type{}, std::false_type{});
-      } else {
-        if (bias_const) epilogue(std::false_type{}, std::true_type{});
-        else epilogue(std::false_type{}, std::false_type{});
-      }
+      auto run = [&](auto mask) {
+        if (bias_const) epilogue(mask, std::true_type{});
+        else epilogue(mask, std::false_type{});
+      };
+      if (!need_mask) run(MaskNo{});
+      else if (GENERIC && mask_is_band(mw0, mw0 + 16 * QT - 1, n0, n0 + C::BN - 1, mc)) run(MaskBand{});
+      else run(MaskGen{});
       // ---- O += P . V  (V rows read transposed by ds_read_b64_tr_b16); the
       // raised wave priority lets this wave's MFMAs issue ahead of the other
       // workgroup's epilogue VALU work on the same SIMD
@@ -1372,6 +1386,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
   if (!seq_ctx(p, /*heavy_last=*/true, sc)) return;
   if (sc.tail > 0) zero_tail<D>(sc, p.N, p.dq, p.dq_rs);
   const int L = sc.L, h = sc.h;
+  if constexpr (GENERIC) prefix_block_first<C::BM>(p, sc);
   const int m0 = sc.blk * C::BM;
   if (m0 >= L) return;
   const MaskCtx mc = mask_ctx(p, sc);
@@ -1482,6 +1497,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
                                   : n0 > mw0 + 31 ? kMaskNone : n0 + C::BN - 1 > mw0 ? kMaskSome : kMaskAll;
     if (wave_active && cls != kMaskNone) {
       const bool need_mask = cls == kMaskSome;
+      const bool band = GENERIC && mask_is_band(mw0, mw0 + 31, n0, n0 + C::BN - 1, mc);
       const bool bias_const = BIAS && (m0 - n0 - (C::BN - 1) >= R1);
       const float* bias_lds = (const float*)(buf + C::BIAS_OFF);
       // Two halves of 32 keys each (key sub-tiles 2c, 2c+1), to keep the
@@ -1506,7 +1522,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
         }
         u32x4 dsa[2];
         auto epilogue = [&](auto masked_tag, auto bconst_tag) {
-          constexpr bool MASKED = decltype(masked_tag)::value;
+          constexpr int MASKED = decltype(masked_tag)::value;
           constexpr bool BCONST = decltype(bconst_tag)::value;
           const float bconst = (BIAS && BCONST) ? bias_lds[0] : 0.f;
           float dacc[4] = {0.f, 0.f, 0.f, 0.f};  // diagonal partial sums (bias gradient)
@@ -1531,7 +1547,9 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
                 float ds = dsilu_dp(t, FP8 ? dp[h2][qt][r] * svv[r] : dp[h2][qt][r]);
                 if constexpr (MASKED) {
                   const int i = mw0 + qt * 16 + li, j = n0 + kt * 16 + 4 * g + r;
-                  const bool ok = GENERIC ? mask_pair(i, j, qid[qt], mask_id(j, mc), mc) : (j <= i);
+                  const bool ok = !GENERIC            ? j <= i
+                                  : MASKED == MaskGen() ? mask_pair(i, j, qid[qt], mask_id(j, mc), mc)
+                                                        : mask_band(i, j, mc);
                   ds = ok ? ds : 0.f;
                 }
                 if constexpr (BIAS) {
@@ -1559,13 +1577,13 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
             else dclampn += dv;
           }
         };
-        if (need_mask) {
-          if (bias_const) epilogue(std::true_type{}, std::true_type{});
-          else epilogue(std::true_type{}, std::false_type{});
-        } else {
-          if (bias_const) epilogue(std::false_type{}, std::true_type{});
-          else epilogue(std::false_type{}, std::false_type{});
-        }
+        auto run = [&](auto mask) {
+          if (bias_const) epilogue(mask, std::true_type{});
+          else epilogue(mask, std::false_type{});
+        };
+        if (!need_mask) run(MaskNo{});
+        else if (GENERIC && band) run(MaskBand{});
+        else run(MaskGen{});
         // ---- dQ += dS . K  (K rows read transposed)
 #pragma unroll
         for (int dt = 0; dt < C::DT; ++dt) {
@@ -2079,7 +2097,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
   // each loop below has a single code path (two paths in one loop push the
   // register allocation past the 256 VGPRs of two waves per SIMD).
   auto tile_body = [&](int t, auto masked_tag, auto bconst_tag) {
-    constexpr bool MASKED = decltype(masked_tag)::value;
+    constexpr int MASKED = decltype(masked_tag)::value;
     constexpr bool BCONST = decltype(bconst_tag)::value;
     const int m0 = tile_m0(t);
     const uint8_t* buf = smem + cur * C::STAGE;
@@ -2137,7 +2155,9 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
             if constexpr (FP8) dval *= sqv[r];
             if constexpr (MASKED) {
               const int i = m0 + qs * 16 + 4 * g + r, j = kw0 + kt * 16 + li;
-              const bool ok = GENERIC ? mask_pair(i, j, mask_id(i, mc), mask_id(j, mc), mc) : (j <= i);
+              const bool ok = !GENERIC            ? j <= i
+                              : MASKED == MaskGen() ? mask_pair(i, j, mask_id(i, mc), mask_id(j, mc), mc)
+                                                    : mask_band(i, j, mc);
               pval = ok ? pval : 0.f;
               dval = ok ? dval : 0.f;
             }
@@ -2190,15 +2210,19 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
 
   int t = 0;
   if constexpr (GENERIC) {
-    // masked tiles (prefix, diagonal), the run of tiles whose pairs are all
-    // valid, then the rest masked (the window's edge)
-    auto all = [&](int u) {
-      const int m0 = tile_m0(u);
-      return mask_class(m0, m0 + C::BMQ - 1, n0, n0 + C::BN - 1, mc) == kMaskAll;
+    // runs of tiles of one kind: general mask (prefix, targets), band (diagonal,
+    // the window's edge), all pairs valid
+    auto kind = [&](int u) {
+      const int m0 = tile_m0(u), m1 = m0 + C::BMQ - 1, n1 = n0 + C::BN - 1;
+      return mask_class(m0, m1, n0, n1, mc) == kMaskAll ? MaskNo()
+             : mask_is_band(m0, m1, n0, n1, mc)         ? MaskBand()
+                                                        : MaskGen();
     };
-    for (; t < ntiles && !all(t); ++t) tile_body(t, std::true_type{}, std::false_type{});
-    for (; t < ntiles && all(t); ++t) tile_body(t, std::false_type{}, std::false_type{});
-    for (; t < ntiles; ++t) tile_body(t, std::true_type{}, std::false_type{});
+    while (t < ntiles) {
+      for (; t < ntiles && kind(t) == MaskGen(); ++t) tile_body(t, MaskGen{}, std::false_type{});
+      for (; t < ntiles && kind(t) == MaskBand(); ++t) tile_body(t, MaskBand{}, std::false_type{});
+      for (; t < ntiles && kind(t) == MaskNo(); ++t) tile_body(t, MaskNo{}, std::false_type{});
+    }
   } else {
     // Tiles [0, t_mask) touch the diagonal of some wave's keys (queries below
     // n0 + BN - 1); tiles from t_const on have every offset i-j >= R-1 and so a
@@ -2206,10 +2230,10 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
     const int t_mask = min(ntiles, (C::BN - 1 + C::BMQ - 1) / C::BMQ);
     int t_const = ntiles;
     if (BIAS) t_const = max(t_mask, min(ntiles, (R1 + C::BN - 1 + C::BMQ - 1) / C::BMQ));
-    for (; t < t_mask; ++t) tile_body(t, std::true_type{}, std::false_type{});
-    for (; t < t_const; ++t) tile_body(t, std::false_type{}, std::false_type{});
+    for (; t < t_mask; ++t) tile_body(t, MaskGen{}, std::false_type{});
+    for (; t < t_const; ++t) tile_body(t, MaskNo{}, std::false_type{});
     if constexpr (BIAS) {
-      for (; t < ntiles; ++t) tile_body(t, std::false_type{}, std::true_type{});
+      for (; t < ntiles; ++t) tile_body(t, MaskNo{}, std::true_type{});
     }
   }
 
@@ -2579,9 +2603,9 @@ __global__ void __launch_bounds__(F8Bwd::NT, 3) hstu_bwd_f8_dkdv_kernel(AttnPara
   if (BIAS) t_const = max(1, min(ntiles, (R1 + 127 + C::BM - 1) / C::BM));
   tile_body(0, std::true_type{}, std::false_type{});
   int t = 1;
-  for (; t < t_const; ++t) tile_body(t, std::false_type{}, std::false_type{});
+  for (; t < t_const; ++t) tile_body(t, MaskNo{}, std::false_type{});
   if constexpr (BIAS) {
-    for (; t < ntiles; ++t) tile_body(t, std::false_type{}, std::true_type{});
+    for (; t < ntiles; ++t) tile_body(t, MaskNo{}, std::true_type{});
   }
 
   fp8_saturate_mode(false);

@@ -313,6 +313,17 @@ __device__ __forceinline__ MaskClass mask_class(int i0, int i1, int j0, int j1, 
   const bool prefix = a0 == 0 && b0 < m.last;
   return diag || near || prefix ? kMaskSome : kMaskNone;
 }
+// Whether positions in the block are the indices themselves (minus c1) and no
+// row is a prefix row: pair (i, j) is then valid when 0 <= i - j <= window,
+// one subtraction and one comparison.  The general test's comparisons meet in
+// scalar registers, several dependent scalar operations an element: with a
+// window of 256 (half of the tiles cut) it was MASK_BAND_NUMBERS
+__device__ __forceinline__ bool mask_is_band(int i0, int i1, int j0, int j1, const MaskCtx& m) {
+  return (m.last == INT_MIN || i0 > m.c1) && min(i0, j0) >= m.c1 && max(i1, j1) - m.c1 <= m.clamp;
+}
+__device__ __forceinline__ bool mask_band(int i, int j, const MaskCtx& m) {
+  return (unsigned)(i - j) <= (unsigned)m.window;
+}
 // First key a row block starting at row m0 (no prefix row) can see.
 __device__ __forceinline__ int mask_first_key(int m0, const MaskCtx& m) {
   const int a = mask_id(m0, m);
