@@ -233,7 +233,6 @@ struct AttnParams {
   int dbias_w;            // floats per row: offsets 0 .. R-1 (causal), -(R-1) .. R-1 (generic masks)
   const int* sched_items;  // block schedule (schedule_block): [8][sched_cap] (sequence*H + head); null: direct grid
   const int* sched_start;  // [8][sched_cap + 1] first block position of each item on its XCD
-  const int* sched_count;  // [8] items per XCD
   int sched_cap;
   int blocks_per_seq;  // ceil(N / 128)
   uint8_t* ds_ws;           // workspace: bf16 dS tiles written by dK/dV, read by dQ (causal masks)
@@ -284,6 +283,11 @@ __device__ __forceinline__ void dbias_store_row(const AttnParams& p, const float
   }
 }
 
+// Items (sequence, head) that schedule_block deals to XCD x (snake order).
+__host__ __device__ inline int sched_items_of(int items, int x) {
+  const int full = items >> 4, rem = items & 15;
+  return 2 * full + (x < rem ? 1 : 0) + (15 - x < rem ? 1 : 0);
+}
 struct SeqCtx {
   int64_t start;
   int L, b, h, blk;
@@ -310,17 +314,26 @@ __device__ __forceinline__ bool seq_ctx(const AttnParams& p, bool heavy_last, Se
     m = u / items;
     bh = u - m * items;
   } else {
-    const int n = p.sched_count[x];
+    // the last of the XCD's n items whose first block is <= k: the lanes look at
+    // 64 of them at once, two dependent loads where a binary search had log2 n
+    // (the masked training batch above, 1 200 short blocks in three kernels:
+    // 242.6 -> 239.2 us)
+    const int lane = threadIdx.x & 63, n = sched_items_of(p.B * p.H, x);
     const int* st = p.sched_start + x * (p.sched_cap + 1);
-    if (k >= st[n]) return false;
-    int lo = 0, hi = n - 1;  // the last item whose first block is <= k
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (st[mid] <= k) lo = mid;
-      else hi = mid - 1;
+    const int total = st[n];
+    int base = 0;
+    for (int c0 = 0; n > 64 && c0 < n; c0 += 64 * 64) {  // the chunk of 64 items
+      const int c = c0 + 64 * lane;
+      const int le = __popcll(__ballot((c < n ? st[c] : INT_MAX) <= k));
+      if (le > 0) base = c0 + 64 * (le - 1);
+      if (le < 64) break;
     }
-    bh = p.sched_items[x * p.sched_cap + lo];
-    m = k - st[lo];
+    const int j = base + lane;
+    const int first = j < n ? st[j] : INT_MAX, item = j < n ? p.sched_items[x * p.sched_cap + j] : 0;
+    if (k >= total) return false;
+    const int at = __popcll(__ballot(first <= k)) - 1;
+    bh = __builtin_amdgcn_readlane(item, at);
+    m = k - __builtin_amdgcn_readlane(first, at);
   }
   c.b = bh / p.H;
   c.h = bh - c.b * p.H;
@@ -2991,15 +3004,14 @@ __device__ void build_bias_ext(const float* bias, int R, int N, float* ext, int 
 // work of a sorted list within one item of even; on an XCD they run in rank
 // order, heaviest first.  One workgroup of 1024 threads; O(B*H) work.
 // Output (ints): items[8][cap], start[8][cap+1] (exclusive block-count
-// prefix per XCD, start[x][n_x] = the XCD's total), count[8]; scratch nb[B],
-// rank[B].
+// prefix per XCD, start[x][n_x] = the XCD's total); scratch nb[B], rank[B].
 // ---------------------------------------------------------------------------
 constexpr int kSchedBins = 1024;  // block counts >= 1023 share the last bin (order only)
 
 __host__ __device__ inline int sched_cap(int B, int H) { return (B * H + 7) / 8; }
 inline int64_t sched_ints(int B, int H) {
   const int64_t cap = sched_cap(B, H);
-  return 8 * cap + 8 * (cap + 1) + 8 + 2 * (int64_t)B;
+  return 8 * cap + 8 * (cap + 1) + 2 * (int64_t)B;
 }
 
 // The time is its barriers and memory round trips, so the counts, ranks and
@@ -3009,12 +3021,12 @@ __device__ void schedule_block(const int64_t* seq_offsets, int B, int H, int N, 
   const int cap = sched_cap(B, H);
   int* items = ws;
   int* start = items + 8 * cap;
-  int* count = start + 8 * (cap + 1);
+  int* scratch = start + 8 * (cap + 1);
   __shared__ int bins[kSchedBins];
   __shared__ int part[kSchedBins / 64];
   __shared__ int nb_lds[kSchedBins], rank_lds[kSchedBins], cnt_lds[4 * kSchedBins];
-  int* nbv = B <= kSchedBins ? nb_lds : count + 8;
-  int* rank = B <= kSchedBins ? rank_lds : count + 8 + B;
+  int* nbv = B <= kSchedBins ? nb_lds : scratch;
+  int* rank = B <= kSchedBins ? rank_lds : scratch + B;
   int* cnt = 8 * (cap + 1) <= 4 * kSchedBins ? cnt_lds : start;  // block count of each XCD's j-th item
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;  // blockDim.x == kSchedBins
   bins[tid] = 0;
@@ -3056,8 +3068,7 @@ __device__ void schedule_block(const int64_t* seq_offsets, int B, int H, int N, 
   __syncthreads();
   // per XCD (one wave each): exclusive scan of the block counts
   if (wave < 8) {
-    const int x = wave, BH = B * H, full = BH >> 4, rem = BH & 15;
-    const int n = 2 * full + (x < rem ? 1 : 0) + (15 - x < rem ? 1 : 0);
+    const int x = wave, n = sched_items_of(B * H, x);
     int* st = start + x * (cap + 1);
     int carry = 0;
     for (int j0 = 0; j0 < n; j0 += 64) {
@@ -3067,10 +3078,7 @@ __device__ void schedule_block(const int64_t* seq_offsets, int B, int H, int N, 
       if (j < n) st[j] = carry + in - c;
       carry += __shfl(in, 63);
     }
-    if (lane == 0) {
-      st[n] = carry;
-      count[x] = n;
-    }
+    if (lane == 0) st[n] = carry;
   }
 }
 
@@ -3094,7 +3102,6 @@ void use_schedule(AttnParams& p, int B, int H, int* ws) {
   p.sched_cap = sched_cap(B, H);
   p.sched_items = ws;
   p.sched_start = ws + 8 * p.sched_cap;
-  p.sched_count = p.sched_start + 8 * (p.sched_cap + 1);
 }
 // workgroups (pairs, for the full-FP8 dK/dV): every XCD's longest possible
 // list, or every block of a direct grid, a multiple of 8

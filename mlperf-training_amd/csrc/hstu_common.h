@@ -315,9 +315,9 @@ __device__ __forceinline__ MaskClass mask_class(int i0, int i1, int j0, int j1, 
 }
 // Whether positions in the block are the indices themselves (minus c1) and no
 // row is a prefix row: pair (i, j) is then valid when 0 <= i - j <= window,
-// one subtraction and one comparison.  The general test's comparisons meet in
-// scalar registers, several dependent scalar operations an element: with a
-// window of 256 (half of the tiles cut) it was MASK_BAND_NUMBERS
+// one subtraction and one comparison (the general test's three comparisons
+// meet in scalar registers, several dependent scalar operations an element).
+// The training batch above, together with the prefix blocks first: 251 -> 243 us.
 __device__ __forceinline__ bool mask_is_band(int i0, int i1, int j0, int j1, const MaskCtx& m) {
   return (m.last == INT_MIN || i0 > m.c1) && min(i0, j0) >= m.c1 && max(i1, j1) - m.c1 <= m.clamp;
 }
