@@ -107,6 +107,37 @@ __device__ __forceinline__ void buf_to_lds(BufRsrc r, uint8_t* lds, uint32_t vof
 // instruction, so the compiler's own wait insertion counts it
 __device__ __forceinline__ void lds_dma_wait() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
+// The LDS DMA as inline assembly, invisible to the compiler (which would
+// otherwise wait for all of them before every LDS read): the waits are the
+// caller's, explicit.  M0 is saved and restored.
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+// make_rsrc's descriptor as four scalar registers
+__device__ __forceinline__ i32x4 rsrc_sgprs(const void* base, uint32_t bytes) {
+  const uint64_t a = (uint64_t)(uintptr_t)base;
+  i32x4 r;
+  r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
+  r[1] = __builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu));  // stride 0
+  r[2] = __builtin_amdgcn_readfirstlane((int)bytes);
+  r[3] = 0x00020000;
+  return r;
+}
+// lane l writes 16 bytes at lds + 16 l from voffset v + soff
+__device__ __forceinline__ void dma_to_lds(uint32_t lds, uint32_t v, i32x4 r, uint32_t soff) {
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "s"(lds), "v"(v), "s"(r), "s"(soff)
+      : "memory");
+}
+// At most VM of this wave's vector-memory operations outstanding and its LDS
+// operations done, then s_barrier.
+template <int VM>
+__device__ __forceinline__ void dma_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(VM) : "memory");
+}
+
 // Transposed LDS read (gfx950 ds_read_b64_tr_b16).  Within each 16-lane
 // group, lane j supplies the address of 4 consecutive bf16 M[j][0..3]; lane i
 // receives M[4r + i/4][i%4] for r = 0..3.  With lane j pointing at row

@@ -769,17 +769,6 @@ constexpr int kDuoThreads = 256;
 constexpr int kDuoItem = 128 * 128;  // 16 KiB
 constexpr int kDuoSlots = 5;         // 80 KiB: two workgroups per CU
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-// make_rsrc's descriptor as four scalar registers, for inline assembly
-__device__ __forceinline__ i32x4 rsrc_sgprs(const void* base, uint32_t bytes) {
-  const uint64_t a = (uint64_t)(uintptr_t)base;
-  i32x4 r;
-  r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
-  r[1] = __builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu));  // stride 0
-  r[2] = __builtin_amdgcn_readfirstlane((int)bytes);
-  r[3] = 0x00020000;
-  return r;
-}
 // 4 x 16 bytes per lane from the buffer to LDS: load j writes lds + 1024 j +
 // 16 lane, from voffset v[j] + soff.  M0 is saved and restored.
 __device__ __forceinline__ void duo_dma4(uint32_t lds, const uint32_t (&v)[4], i32x4 r, uint32_t soff) {
@@ -795,23 +784,6 @@ __device__ __forceinline__ void duo_dma4(uint32_t lds, const uint32_t (&v)[4], i
       : "s"(lds), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "s"(r), "s"(soff)
       : "memory", "scc");
 }
-// one of those loads: lane l writes lds + 16 l from voffset v + soff
-__device__ __forceinline__ void duo_dma1(uint32_t lds, uint32_t v, i32x4 r, uint32_t soff) {
-  uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "s"(lds), "v"(v), "s"(r), "s"(soff)
-      : "memory");
-}
-// At most VM of this wave's vector-memory operations outstanding and its LDS
-// operations done, then s_barrier.
-template <int VM>
-__device__ __forceinline__ void duo_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(VM) : "memory");
-}
-
 template <bool E4M3_OUT, bool RESID, bool A_BF8>
 __global__ void __launch_bounds__(kDuoThreads, 2) fp8_gemm_duo_kernel(GemmParams p, int per_xcd) {
   __shared__ __attribute__((aligned(1024))) uint8_t ring[kDuoSlots][kDuoItem];
@@ -924,8 +896,8 @@ __global__ void __launch_bounds__(kDuoThreads, 2) fp8_gemm_duo_kernel(GemmParams
     constexpr bool FIRST = decltype(first_c)::value, LAST = decltype(last_c)::value;
     // this wave's items of step s have landed (issued after them: items
     // 3 s + 3, 3 s + 4, if step s + 1 exists), then every wave's
-    if constexpr (LAST) duo_barrier<0>();
-    else duo_barrier<8>();
+    if constexpr (LAST) dma_barrier<0>();
+    else dma_barrier<8>();
     const uint8_t* sa_ = ring[(3 * s) % kDuoSlots];
     const uint8_t* sw_ = ring[(3 * s + 1 + (wave >> 1)) % kDuoSlots] + w_off;
     i32x8 w[4], a0[4], a1[4];
@@ -937,7 +909,7 @@ __global__ void __launch_bounds__(kDuoThreads, 2) fp8_gemm_duo_kernel(GemmParams
     read_a(sa_, 0, a0);
     mfma_rows(w, a0, 0, FIRST);
     read_a(sa_, 4, a1);
-    duo_barrier<0>();  // every wave has read step s: its three slots are free
+    dma_barrier<0>();  // every wave has read step s: its three slots are free
     if constexpr (LAST) {
       load_consts();
     } else {
@@ -1116,8 +1088,8 @@ __global__ void __launch_bounds__(kDuoThreads, 2) bf16_gemm_duo_kernel(GemmParam
   // of loads) before its next MFMA.
   auto kstep = [&](int s, auto items_c) {
     constexpr int ITEMS = decltype(items_c)::value;
-    if constexpr (ITEMS == 0) duo_barrier<0>();
-    else duo_barrier<8>();
+    if constexpr (ITEMS == 0) dma_barrier<0>();
+    else dma_barrier<8>();
     const uint8_t* sa_ = ring[(3 * s) % kDuoSlots];
     const uint8_t* sw_ = ring[(3 * s + 1 + (wave >> 1)) % kDuoSlots] + w_off;
     u32x4 w[2][4], a[4][4];
@@ -1138,9 +1110,9 @@ __global__ void __launch_bounds__(kDuoThreads, 2) bf16_gemm_duo_kernel(GemmParam
       if constexpr ((n & 1) == 1 && (n >> 1) < 4 * ITEMS) {  // items 3 s + 5 (W1), 3 s + 6 (A), 3 s + 7 (W0)
         constexpr int k = n >> 3, j = (n >> 1) & 3;
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (k == 0) duo_dma1(dst[0] + 1024 * j, wv[1][j], wrs, kw1);
-        else if constexpr (k == 1) duo_dma1(dst[1] + 1024 * j, av[j], ars, ka);
-        else duo_dma1(dst[2] + 1024 * j, wv[0][j], wrs, ka);
+        if constexpr (k == 0) dma_to_lds(dst[0] + 1024 * j, wv[1][j], wrs, kw1);
+        else if constexpr (k == 1) dma_to_lds(dst[1] + 1024 * j, av[j], ars, ka);
+        else dma_to_lds(dst[2] + 1024 * j, wv[0][j], wrs, ka);
         __builtin_amdgcn_sched_barrier(0);
       }
     });
@@ -1273,9 +1245,9 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_few_rows_kernel(GemmParams p
   auto issue = [&](int s) {  // four loads of this wave: A, A, W, W
     const uint32_t dst = __builtin_amdgcn_readfirstlane(ring0 + (uint32_t)((s % kFewStages) * kFewStage + 2048 * wave));
 #pragma unroll
-    for (int j = 0; j < 2; ++j) duo_dma1(dst + 1024 * j, av[j], ars, (uint32_t)(128 * s));
+    for (int j = 0; j < 2; ++j) dma_to_lds(dst + 1024 * j, av[j], ars, (uint32_t)(128 * s));
 #pragma unroll
-    for (int j = 0; j < 2; ++j) duo_dma1(dst + kFewStage / 2 + 1024 * j, wv[j], wrs, (uint32_t)(128 * s));
+    for (int j = 0; j < 2; ++j) dma_to_lds(dst + kFewStage / 2 + 1024 * j, wv[j], wrs, (uint32_t)(128 * s));
   };
   for (int s = 0; s < min(kFewStages - 1, nk); ++s) issue(s);
 
@@ -1288,7 +1260,7 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_few_rows_kernel(GemmParams p
   auto kstep = [&](int s, auto vm_c) {
     // step s has landed when only the loads of the (up to two) later steps
     // issued so far are outstanding
-    duo_barrier<decltype(vm_c)::value>();
+    dma_barrier<decltype(vm_c)::value>();
     if (s + kFewStages - 1 < nk) issue(s + kFewStages - 1);
     const uint8_t* sa_ = ring[s % kFewStages] + wm * 128;
     const uint8_t* sw_ = ring[s % kFewStages] + kFewStage / 2 + wn * 128;

@@ -13,33 +13,43 @@
 // Design: the output is small (0.75-1 M elements) and the contraction long
 // (T ~ 162 K tokens), so the tokens are split over workgroups: tiles x split
 // ~ one workgroup per CU.  A workgroup owns a 256 (n1) x 256 (n2) tile of one
-// token range; 8 waves as 4 (n1) x 2 (n2) of 64 x 128.  Each k-step of 32
-// tokens stages both operands' 32 x 512-byte tile rows in LDS as they lie in
-// memory (token rows, 544-byte pitch), and the MFMA operands come out of LDS
-// with the transposed read ds_read_b64_tr_b16, which turns a token-major tile
-// into k(token)-contiguous fragments: lane group g gets tokens {4g..4g+3,
-// 16+4g..16+4g+3} of column li in both operands, so the contraction sees the
-// same token order on both sides.  The MFMA (v_mfma_f32_16x16x32_bf16) runs
-// with B as its A operand, so a lane's result is 4 consecutive n2 of one n1
-// row.  Global loads for step k+1 are issued into registers before step k's
-// MFMAs and written to the other LDS buffer after them (one barrier per
-// step).  Workgroups are numbered so that the tiles of one token range run on
-// one XCD and share its L2.  With split > 1 every workgroup writes an fp32
-// partial tile; a second kernel sums the splits in a fixed order, applies
-// sa * sb and writes bf16 or fp32 (bitwise reproducible, no atomics).
-// Optionally (bf16) the workgroups of the first n1 tile also sum B's columns
-// from the registers they stage (the projection's bias gradient), so the
-// layer needs no separate pass over d(uvqk) for it.
-// The fp8 form (e4m3 A, e4m3 or e5m2 B: the reference's fp8_wgrad operands)
-// takes 128-token steps of 256-byte rows through the same LDS budget, reads
-// its fragments with ds_read_b64_tr_b8 (four 8-token reads per 32-byte
-// fragment) and runs v_mfma_f32_16x16x128_f8f6f4 with the operands' formats.
+// token range; 8 waves as 4 (n1) x 2 (n2) of 64 x 128.  Token rows lie in LDS
+// as in memory, and the MFMA operands come out with the transposed reads
+// (ds_read_b64_tr_b16, _b8), which turn a token-major tile into
+// k(token)-contiguous fragments with the same token order in both operands.
+// The MFMA (v_mfma_f32_16x16x32_bf16, 16x16x128_f8f6f4) runs with B as its A
+// operand, so a lane's result is 4 consecutive n2 of one n1 row.
+// What bounds it: the matrix cores and, close behind, the transposed reads (for
+// fp8 1 900 LDS cycles against 2 050 MFMA cycles a step), so the two must
+// overlap although the eight waves meet at a barrier every step: the
+// fragments roll.  A fragment's registers are refilled with the next step's as
+// soon as its last MFMA is issued, so the LDS reads of step k + 1 run under the
+// MFMAs of step k, and step k's LDS buffer is already free while its MFMAs run:
+// LDS DMA (inline assembly, explicit waits, spread between the MFMAs) fills it
+// with the step that comes a whole ring later.  One barrier per step.
+// Rows are unpadded; 16-byte chunk c of row r sits at c ^ swz(r), which spreads
+// the transposed reads over all banks.
+// Measured, product + second pass, against operands loaded through registers and
+// read from padded LDS all at once behind the barrier, in us:
+//                        512 x 2048        1536 x 512
+//   bf16 T = 162 251   361.5 -> 346.0    254.1 -> 231.7  (983 / 1 101 TFLOP/s)
+//   bf16 T =  37 429    99.9 ->  91.5     73.7 ->  67.7
+//   fp8  T = 162 251   176.5 -> 175.0    133.5 -> 135.0  (no gain: one code for
+//   fp8  T =  37 429    57.6 ->  57.5     47.5 ->  47.7   both formats)
+// Workgroups are numbered so that the tiles of one token range run on one XCD
+// and share its L2.  With split > 1 every workgroup writes an fp32 partial
+// tile; a second kernel sums the splits in a fixed order, applies sa * sb and
+// writes bf16 or fp32 (bitwise reproducible, no atomics).  Optionally (bf16)
+// the workgroups of the first n1 tile also sum B's columns from LDS (the
+// projection's bias gradient), so the layer needs no separate pass over
+// d(uvqk) for it.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "hstu_common.h"
@@ -52,20 +62,21 @@ constexpr int kWThreads = 512;  // 8 waves
 constexpr int kBN1 = 256, kBN2 = 256;  // output tile
 constexpr int kCus = 256;
 
-// Per operand format: bf16 steps of 64 tokens (512-byte tile rows, 544-byte
-// pitch) or fp8 steps of 128 tokens (256-byte rows, 272-byte pitch).  Both
-// stage 64 KiB per step and take 136 KiB of LDS for two steps.
+// Per operand format: bf16 steps of 32 tokens (512-byte tile rows) in a ring of
+// four, fp8 steps of 128 tokens (256-byte rows) in a ring of two: 128 KiB.
 template <bool F8>
 struct WCfg {
-  static constexpr int KT = F8 ? 128 : 64;           // tokens per k-step
-  static constexpr int ES = F8 ? 1 : 2;              // bytes per element
-  static constexpr int ROW = kBN1 * ES;              // tile row bytes
-  static constexpr int PITCH = ROW + (F8 ? 16 : 32);  // conflict-free transposed reads
-  static constexpr int TILE = KT * PITCH;
-  static constexpr int STAGE = 2 * TILE;             // A tile then B tile
-  static constexpr int LDS = 2 * STAGE;
-  static constexpr int CPR = ROW / 16;               // 16-byte chunks per tile row
-  static constexpr int Q = KT * CPR / kWThreads;     // staged chunks per thread per operand
+  static constexpr int KT = F8 ? 128 : 32;  // tokens per k-step
+  static constexpr int RING = F8 ? 2 : 4;
+  static constexpr int ES = F8 ? 1 : 2;     // bytes per element
+  static constexpr int ROW = kBN1 * ES;     // tile row bytes
+  static constexpr int TILE = KT * ROW;
+  static constexpr int STAGE = 2 * TILE;    // A tile then B tile
+  static constexpr int LDS = RING * STAGE;
+  static constexpr int CPR = ROW / 16;      // 16-byte chunks per tile row
+  static constexpr int NDMA = TILE / 1024 / 8;  // loads per wave and operand
+  // bf16: a pass of a transposed read takes 8 rows x 2 chunks; fp8: 16 rows x 1
+  __host__ __device__ static constexpr int swz(int r) { return F8 ? r & 15 : 2 * (r & 7); }
 };
 constexpr int kWLds = WCfg<false>::LDS;
 static_assert(WCfg<true>::LDS == kWLds, "one LDS size");
@@ -93,8 +104,8 @@ struct WgradParams {
 template <bool F8, int FA, int FB>
 __global__ void __launch_bounds__(kWThreads, 1) wgrad_kernel(WgradParams p) {
   using C = WCfg<F8>;
-  constexpr int kKT = C::KT, kWPitch = C::PITCH, kWTile = C::TILE, kWStage = C::STAGE, kQ = C::Q;
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  constexpr int kKT = C::KT;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   // XCD-contiguous numbering: workgroup b runs on XCD b % 8; consecutive idx
   // (one token range, all its tiles) land on one XCD.
   const int total = p.tiles * p.split;
@@ -108,52 +119,52 @@ __global__ void __launch_bounds__(kWThreads, 1) wgrad_kernel(WgradParams p) {
   const int64_t te = min(tb + p.tps, p.T);
   const int nk = (int)((te - tb + kKT - 1) / kKT);
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15,
+            g = lane >> 4;
   const int w1 = (wave >> 1) * 64, w2 = (wave & 1) * 128;
 
   // Token rows tb .. te-1 of the tile's column band; rows past te (the next
   // split's, or past T) read as zero.
   const uint32_t lda = (uint32_t)p.lda, ldb = (uint32_t)p.ldb;
-  const BufRsrc ar = make_rsrc(p.A + tb * p.lda + n10 * C::ES, (uint32_t)((te - tb - 1) * p.lda + C::ROW));
-  const BufRsrc br = make_rsrc(p.B + tb * p.ldb + n20 * C::ES, (uint32_t)((te - tb - 1) * p.ldb + C::ROW));
-  // staging: chunk c = tid + 512 q (q < kQ) of a kKT-row tile
-  uint32_t va[kQ], vb[kQ], lo[kQ];
+  const uint32_t a_bytes = (uint32_t)((te - tb - 1) * p.lda + C::ROW), b_bytes = (uint32_t)((te - tb - 1) * p.ldb + C::ROW);
+  const i32x4 ar = rsrc_sgprs(p.A + tb * p.lda + n10 * C::ES, a_bytes);
+  const i32x4 br = rsrc_sgprs(p.B + tb * p.ldb + n20 * C::ES, b_bytes);
+  // LDS slot q = 64 i + lane of a tile is row q / CPR, position q % CPR
+  uint32_t va[C::NDMA], vb[C::NDMA];
 #pragma unroll
-  for (int q = 0; q < kQ; ++q) {
-    const int c = tid + kWThreads * q, row = c / C::CPR, col = c % C::CPR;
-    va[q] = row * lda + col * 16;
-    vb[q] = row * ldb + col * 16;
-    lo[q] = row * kWPitch + col * 16;
+  for (int j = 0; j < C::NDMA; ++j) {
+    const int q = 64 * (C::NDMA * wave + j) + lane, row = q / C::CPR, ch = (q % C::CPR) ^ C::swz(row);
+    va[j] = row * lda + ch * 16;
+    vb[j] = row * ldb + ch * 16;
   }
-  u32x4 ra[kQ], rb[kQ];
-  auto load = [&](int kk) {
-    const uint32_t sa_off = (uint32_t)kk * kKT * lda, sb_off = (uint32_t)kk * kKT * ldb;
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) {
-      ra[q] = buf_ld128(ar, va[q], sa_off);
-      rb[q] = buf_ld128(br, vb[q], sb_off);
-    }
+  const uint32_t lds0 =
+      __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)smem);
+  // load i (0 .. 2 NDMA - 1) of step kk; steps past the range read zeros: the
+  // range check takes the vector offset against the records less the scalar
+  // offset, which therefore never exceeds the records
+  auto issue = [&](int kk, auto i_c) {
+    constexpr int i = decltype(i_c)::value, j = i % C::NDMA;
+    const uint32_t dst = lds0 + (uint32_t)((kk % C::RING) * C::STAGE) + 1024u * (uint32_t)(C::NDMA * wave + j);
+    if constexpr (i < C::NDMA) dma_to_lds(dst, va[j], ar, kk < nk ? (uint32_t)kk * kKT * lda : a_bytes);
+    else dma_to_lds(dst + C::TILE, vb[j], br, kk < nk ? (uint32_t)kk * kKT * ldb : b_bytes);
   };
-  // column sums of B (the bias gradient of the layer's projection), taken
-  // from the staged registers by the workgroups of the first n1 tile: a
-  // thread's chunks all sit at byte column 16 (tid % 32) of the tile
+
+  // column sums of B (the bias gradient of the layer's projection) by the
+  // workgroups of the first n1 tile: thread tid sums chunk tid % 32 of rows
+  // tid / 32 + 16 q of every step
   const bool do_cs = !F8 && p.colsum != nullptr && t1 == 0;
   float cs[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  auto store = [&](uint8_t* st) {
+  auto add_cols = [&](const uint8_t* bt) {
 #pragma unroll
-    for (int q = 0; q < kQ; ++q) {
-      *(u32x4*)(st + lo[q]) = ra[q];
-      *(u32x4*)(st + kWTile + lo[q]) = rb[q];
-    }
-    if (do_cs) {
+    for (int q = 0; q < kKT / 16; ++q) {
+      const int row = (tid >> 5) + 16 * q;
+      const u32x4 v = lds_ld128(bt + row * C::ROW + (((tid & 31) ^ C::swz(row)) * 16));
 #pragma unroll
-      for (int q = 0; q < kQ; ++q)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t w = rb[q][e];
-          cs[2 * e] += __builtin_bit_cast(float, w << 16);
-          cs[2 * e + 1] += __builtin_bit_cast(float, w & 0xffff0000u);
-        }
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t w = v[e];
+        cs[2 * e] += __builtin_bit_cast(float, w << 16);
+        cs[2 * e + 1] += __builtin_bit_cast(float, w & 0xffff0000u);
+      }
     }
   };
 
@@ -163,59 +174,65 @@ __global__ void __launch_bounds__(kWThreads, 1) wgrad_kernel(WgradParams p) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[j][i] = zero4();
 
-  if (nk > 0) {
-    load(0);
-    store(smem);
-  }
-  __syncthreads();
-  // transposed-read start.  bf16: row 4g + li/4, 4-column group li % 4.
-  // fp8: token row 8g + li/2 (plus 32 per read), 8-column half li % 2.
-  const int tr = F8 ? (8 * g + (li >> 1)) * kWPitch + (li & 1) * 8 : (4 * g + (li >> 2)) * kWPitch + (li & 3) * 8;
-  const int a_rd = tr + w1 * C::ES, b_rd = kWTile + tr + w2 * C::ES;
-  for (int kk = 0; kk < nk; ++kk) {
-    const uint8_t* buf = smem + (kk & 1) * kWStage;
-    if (kk + 1 < nk) load(kk + 1);
+  // Transposed reads of column block c0 (16 columns).  bf16: lane (li, g) of
+  // the two reads addresses token rows 4g + li/4 (+16), columns 4 (li % 4); fp8:
+  // rows 8g + li/2 (+32 per read, four reads), columns 8 (li % 2); a lane then
+  // holds the same tokens of its column in both operands.
+  const int r0 = F8 ? 8 * g + (li >> 1) : 4 * g + (li >> 2);
+  const int in0 = F8 ? (li & 1) * 8 : (li & 1) * 8, ch0 = F8 ? 0 : (li >> 1) & 1;
+  const int rd0 = r0 * C::ROW + in0, sw0 = (ch0 ^ C::swz(r0)) * 16;
+  using Frag = std::conditional_t<F8, i32x8, u32x4>;
+  auto frag = [&](const uint8_t* t, int c0) {  // c0 * ES is a multiple of 16 (fp8) or 32 (bf16) bytes
+    const uint8_t* q = t + rd0 + ((c0 * C::ES) ^ sw0);
     if constexpr (F8) {
-      // one 128-token MFMA step: lane (li, g) holds tokens 32r + 8g .. +7 of
-      // its column in bytes 8r .. 8r+7 (r = 0..3), the same in both operands
-      auto frag = [&](const uint8_t* q0) {
-        const u32x2 r0 = lds_tr8(q0), r1 = lds_tr8(q0 + 32 * kWPitch);
-        const u32x2 r2 = lds_tr8(q0 + 64 * kWPitch), r3 = lds_tr8(q0 + 96 * kWPitch);
-        i32x8 f;
-        f[0] = (int)r0[0]; f[1] = (int)r0[1]; f[2] = (int)r1[0]; f[3] = (int)r1[1];
-        f[4] = (int)r2[0]; f[5] = (int)r2[1]; f[6] = (int)r3[0]; f[7] = (int)r3[1];
-        return f;
-      };
-      i32x8 af[4], bfr[8];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) af[i] = frag(buf + a_rd + 16 * i);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) bfr[j] = frag(buf + b_rd + 16 * j);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          acc[j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bfr[j], af[i], acc[j][i], FB, FA, 0, 0, 0, 0);
+      const u32x2 x0 = lds_tr8(q), x1 = lds_tr8(q + 32 * C::ROW);
+      const u32x2 x2 = lds_tr8(q + 64 * C::ROW), x3 = lds_tr8(q + 96 * C::ROW);
+      i32x8 f;
+      f[0] = (int)x0[0]; f[1] = (int)x0[1]; f[2] = (int)x1[0]; f[3] = (int)x1[1];
+      f[4] = (int)x2[0]; f[5] = (int)x2[1]; f[6] = (int)x3[0]; f[7] = (int)x3[1];
+      return f;
     } else {
-#pragma unroll
-    for (int h = 0; h < kKT / 32; ++h) {
-      const uint8_t* hb = buf + h * 32 * kWPitch;
-      u32x4 af[4], bfr[8];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        af[i] = cat_tr(lds_tr16(hb + a_rd + 32 * i), lds_tr16(hb + a_rd + 32 * i + 16 * kWPitch));
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        bfr[j] = cat_tr(lds_tr16(hb + b_rd + 32 * j), lds_tr16(hb + b_rd + 32 * j + 16 * kWPitch));
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[j][i] = mfma_bf16(bfr[j], af[i], acc[j][i]);
+      return cat_tr(lds_tr16(q), lds_tr16(q + 16 * C::ROW));
     }
-    }
-    if (kk + 1 < nk) store(smem + ((kk + 1) & 1) * kWStage);
-    __syncthreads();
+  };
+  Frag af[4], bfr[8];
+  if (nk > 0) {
+    static_for<C::RING>([&](auto k_c) {
+      static_for<2 * C::NDMA>([&](auto i_c) { issue(decltype(k_c)::value, i_c); });
+    });
+    dma_barrier<(C::RING - 1) * 2 * C::NDMA>();  // step 0 has landed
+#pragma unroll
+    for (int i = 0; i < 4; ++i) af[i] = frag(smem, w1 + 16 * i);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) bfr[j] = frag(smem + C::TILE, w2 + 16 * j);
+    if (do_cs) add_cols(smem + C::TILE);
   }
+  for (int kk = 0; kk < nk; ++kk) {
+    // step kk + 1 has landed (steps kk + 2 .. kk + RING - 1 may be in flight),
+    // and every wave has read step kk: its buffer takes step kk + RING
+    dma_barrier<(C::RING - 2) * 2 * C::NDMA>();
+    const uint8_t* nb = smem + ((kk + 1) % C::RING) * C::STAGE;
+    static_for<8>([&](auto j_c) {
+      constexpr int j = decltype(j_c)::value;
+      static_for<4>([&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        if constexpr (F8)
+          acc[j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bfr[j], af[i], acc[j][i], FB, FA, 0, 0, 0, 0);
+        else
+          acc[j][i] = mfma_bf16(bfr[j], af[i], acc[j][i]);
+        if constexpr (j == 7) af[i] = frag(nb, w1 + 16 * i);
+      });
+      bfr[j] = frag(nb + C::TILE, w2 + 16 * j);
+      if constexpr (j < 2 * C::NDMA) {
+        // bf16 always issues (past the range: zeros), so that the wait counts
+        // hold; fp8 waits for everything
+        if (!F8 || kk + C::RING < nk) issue(kk + C::RING, j_c);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if (do_cs && kk + 1 < nk) add_cols(nb + C::TILE);
+  }
+  dma_barrier<0>();  // nothing in flight to LDS below, or past the workgroup's end
 
   if (do_cs) {
     // fold the 16 row slots (tid / 32) of each column in LDS, in a fixed order

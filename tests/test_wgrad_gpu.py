@@ -122,3 +122,31 @@ def test_wgrad_full_size_against_fp32_library_product(hip_lib, n1, n2):
     ref8 = torch.mm(a8.float().t(), b8.float())
     out8 = fp8_wgrad(a8, b8, one, one, out_dtype=torch.float32)
     assert float((out8 - ref8).norm() / ref8.norm()) <= 1e-4
+
+
+@pytest.mark.parametrize("T,split", [(31, 1), (32, 1), (33, 1), (64, 1), (97, 1), (128, 1), (129, 1), (161, 1), (255, 1),
+                                     (256, 1), (257, 1), (385, 1), (513, 1), (300, 9), (1025, 2)])
+def test_wgrad_ring_edges(hip_lib, T, split):
+    """Token counts at the edges of the kernel's steps (32 tokens for bf16, 128
+    for fp8) and of the rings of steps in flight (4 and 2), one split and
+    several: bf16 with the column sums, e4m3 x e5m2.  Small whole numbers, whose
+    products and sums are exact in fp32 in any order, so the results are equal
+    to the float64 product; rows past T belong to another tensor and hold NaN."""
+    from hstu_amd.wgrad import fp8_wgrad, wgrad
+
+    g = torch.Generator(device="cuda").manual_seed(T)
+    n1, n2 = 512, 256
+    one = torch.ones(1, device="cuda")
+
+    def whole(n, dt):
+        big = torch.full((T + 128, n), float("nan"), device="cuda")
+        big[:T] = torch.randint(-4, 5, (T, n), device="cuda", generator=g).float()
+        return big.to(dt)[:T]
+
+    a, b = whole(n1, torch.bfloat16), whole(n2, torch.bfloat16)
+    out, cs = wgrad(a, b, out_dtype=torch.float32, split=split, with_colsum=True)
+    assert torch.equal(out.double().cpu(), O.wgrad(a, b))
+    assert torch.equal(cs.double().cpu(), b.double().cpu().sum(0))
+    a8, b8 = whole(n1, torch.float8_e4m3fn), whole(n2, torch.float8_e5m2)
+    out8 = fp8_wgrad(a8, b8, one, one, out_dtype=torch.float32, split=split)
+    assert torch.equal(out8.double().cpu(), O.wgrad(a8, b8, 1.0, 1.0))
