@@ -1402,7 +1402,8 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
   if constexpr (GENERIC) prefix_block_first<C::BM>(p, sc);
   const int m0 = sc.blk * C::BM;
   if (m0 >= L) return;
-  const MaskCtx mc = mask_ctx(p, sc);
+  MaskCtx mc = mask_ctx(p, sc);
+  if constexpr (BIAS) mc.rows = sc.L;
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15,
             g = lane >> 4;
@@ -1945,7 +1946,8 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
   const int L = sc.L, h = sc.h;
   const int n0 = sc.blk * C::BN;
   if (n0 >= L) return;
-  const MaskCtx mc = mask_ctx(p, sc);
+  MaskCtx mc = mask_ctx(p, sc);
+  if constexpr (BIAS) mc.rows = sc.L;
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15,
             g = lane >> 4;

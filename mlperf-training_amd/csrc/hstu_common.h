@@ -312,7 +312,12 @@ struct MaskCtx {
   int c1;      // contextual_seq_len - 1, or 0 without a prefix
   int clamp;   // position of the targets, INT_MAX without targets
   int window;  // max_attn_len, INT_MAX without
-  int last;    // prefix rows see keys of positions below this (0 without a prefix: none)
+  int last;    // prefix rows see keys of positions below this (INT_MIN without a prefix: none)
+  // Rows from here on have no valid pair: L where a kernel must not take rows
+  // past the sequence for valid (the backward's kernels with a bias: a row past
+  // it is zero, but an infinite or NaN bias at an offset that no pair of the
+  // sequence has would make its products NaN), INT_MAX elsewhere (no test).
+  int rows = INT_MAX;
 };
 __device__ __forceinline__ MaskCtx mask_make(int L, const int32_t* num_targets, int b, int max_attn_len, int ctx) {
   MaskCtx m;
@@ -326,7 +331,8 @@ __device__ __forceinline__ MaskCtx mask_make(int L, const int32_t* num_targets, 
 __device__ __forceinline__ int mask_id(int x, const MaskCtx& m) { return min(max(x - m.c1, 0), m.clamp); }
 // The mask of a pair with positions a = id(i), b = id(j).
 __device__ __forceinline__ bool mask_pair(int i, int j, int a, int b, const MaskCtx& m) {
-  return (i == j) | ((unsigned)(a - b - 1) < (unsigned)m.window) | ((a == 0) & (b < m.last));
+  const bool v = (i == j) | ((unsigned)(a - b - 1) < (unsigned)m.window) | ((a == 0) & (b < m.last));
+  return m.rows == INT_MAX ? v : v & (i < m.rows);
 }
 // What the mask leaves of rows i0 .. i1 against keys j0 .. j1: kMaskNone only
 // if no pair is valid, kMaskAll only if every pair is (then j1 < i0, so no
@@ -338,19 +344,19 @@ __device__ __forceinline__ bool mask_pair(int i, int j, int a, int b, const Mask
 enum MaskClass { kMaskNone = 0, kMaskSome = 1, kMaskAll = 2 };
 __device__ __forceinline__ MaskClass mask_class(int i0, int i1, int j0, int j1, const MaskCtx& m) {
   const int a0 = mask_id(i0, m), a1 = mask_id(i1, m), b0 = mask_id(j0, m), b1 = mask_id(j1, m);
-  if (a0 > b1 && a1 - b0 <= m.window) return kMaskAll;
+  if (a0 > b1 && a1 - b0 <= m.window && i1 < m.rows) return kMaskAll;
   const bool diag = i0 <= j1 && j0 <= i1;
   const bool near = a1 > b0 && a0 - b1 <= m.window;
   const bool prefix = a0 == 0 && b0 < m.last;
   return diag || near || prefix ? kMaskSome : kMaskNone;
 }
-// Whether positions in the block are the indices themselves (minus c1) and no
-// row is a prefix row: pair (i, j) is then valid when 0 <= i - j <= window,
+// Whether positions in the block are the indices themselves (minus c1), no row
+// is a prefix row and none is past m.rows: pair (i, j) is then valid when 0 <= i - j <= window,
 // one subtraction and one comparison (the general test's three comparisons
 // meet in scalar registers, several dependent scalar operations an element).
 // The training batch above, together with the prefix blocks first: 251 -> 243 us.
 __device__ __forceinline__ bool mask_is_band(int i0, int i1, int j0, int j1, const MaskCtx& m) {
-  return (m.last == INT_MIN || i0 > m.c1) && min(i0, j0) >= m.c1 && max(i1, j1) - m.c1 <= m.clamp;
+  return i1 < m.rows && (m.last == INT_MIN || i0 > m.c1) && min(i0, j0) >= m.c1 && max(i1, j1) - m.c1 <= m.clamp;
 }
 __device__ __forceinline__ bool mask_band(int i, int j, const MaskCtx& m) {
   return (unsigned)(i - j) <= (unsigned)m.window;

@@ -179,6 +179,31 @@ def test_generic_mask_tiles(hip_lib, win, ctx, nts, D, with_bias):
         assert orc.rel_l2(db, bd.grad.double().cpu()) <= 1e-2
 
 
+@pytest.mark.parametrize("win,ctx,nts,D", [(0, 0, [0, 64], 64), (500, 0, None, 128), (0, 33, [7, 0], 128), (0, 2, None, 64)])
+def test_generic_mask_bias_past_the_sequence(hip_lib, win, ctx, nts, D):
+    """A bias that is infinite or NaN at offsets that no pair has: the rows of
+    the last tile past a sequence would meet it, and change nothing.  The bytes
+    of a bias that is 0 there."""
+    ops = _ops()
+    H, N, R = 2, 448, 448
+    q, k, v, offs = _case([385, 130], H, D, seed=win + ctx)
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16).to(DEV)
+    nt = None if nts is None else torch.tensor(nts, dtype=torch.int64, device=DEV)
+    res = []
+    for far in (0.0, float("inf"), float("nan")):
+        bias = orc.make_bias(H, R, seed=2, std=0.3)
+        off = torch.arange(2 * R - 1) - (R - 1)
+        bias[:, off.abs() >= 385] = far
+        qd, kd, vd, bd = (t.to(DEV).requires_grad_(True) for t in (q, k, v, bias))
+        out = ops.triton_hstu_mha(N, 0.15, qd, kd, vd, offs.to(DEV), nt, win, ctx, attn_bias=bd)
+        out.backward(dout)
+        res.append([out.detach(), qd.grad, kd.grad, vd.grad, bd.grad])
+    torch.cuda.synchronize()
+    for other in res[1:]:
+        for name, a, b in zip(("out", "dq", "dk", "dv", "dbias"), res[0], other):
+            assert bool(torch.isfinite(a).all()) and torch.equal(a, b), name
+
+
 def test_strided_uvqk_views(hip_lib):
     """q/k/v read in place as column slices of a fused [T, 2048] buffer, and
     dq/dk/dv written into strided views of a fused gradient buffer."""
