@@ -3013,7 +3013,7 @@ constexpr int kSchedBins = 1024;  // block counts >= 1023 share the last bin (or
 __host__ __device__ inline int sched_cap(int B, int H) { return (B * H + 7) / 8; }
 inline int64_t sched_ints(int B, int H) {
   const int64_t cap = sched_cap(B, H);
-  return 8 * cap + 8 * (cap + 1) + 2 * (int64_t)B;
+  return 8 * cap + 8 * (cap + 1) + 8 + 2 * (int64_t)B;  // 8 unused: the size that callers know
 }
 
 // The time is its barriers and memory round trips, so the counts, ranks and
@@ -3146,7 +3146,7 @@ BwdWs bwd_ws(int dtype, int64_t T, int B, int H, int D, int N, int R) {
   w.chunks = o;
   if (R > 0) o += dbias_chunks_bytes(H, R);
   w.dq_base = o;
-  o += align256(((int64_t)B + 1) * 8);
+  o += 2 * align256(((int64_t)B + 1) * 8);  // the second part unused: the size that callers know
   w.ds = o;
   o += ds_tiles_bound(T, B, N) * H * kDsTileBytes;
   w.total = o;
@@ -3788,6 +3788,7 @@ F8Ws f8_ws(int64_t T, int B, int H, int N, int R) {
   o += align256(((int64_t)B + 1) * 8);
   w.maxv = o;
   o += align256(kScaleParts * 2 * 4);
+  o += align256(((int64_t)B + 1) * 8);  // unused: the size that callers know
   w.tiles = o;
   o += f8_tiles_bound(T, B, N) * H * F8Bwd::TILE;
   w.total = o;
