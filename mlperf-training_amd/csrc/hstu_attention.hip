@@ -1947,7 +1947,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
   const int n0 = sc.blk * C::BN;
   if (n0 >= L) return;
   MaskCtx mc = mask_ctx(p, sc);
-  if constexpr (BIAS) mc.rows = sc.L;
+  mc.rows = sc.L;
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15,
             g = lane >> 4;

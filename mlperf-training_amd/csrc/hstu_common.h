@@ -314,9 +314,10 @@ struct MaskCtx {
   int window;  // max_attn_len, INT_MAX without
   int last;    // prefix rows see keys of positions below this (INT_MIN without a prefix: none)
   // Rows from here on have no valid pair: L where a kernel must not take rows
-  // past the sequence for valid (the backward's kernels with a bias: a row past
-  // it is zero, but an infinite or NaN bias at an offset that no pair of the
-  // sequence has would make its products NaN), INT_MAX elsewhere (no test).
+  // past the sequence for valid, INT_MAX elsewhere (no test).  Such a row is
+  // zero, but its products with an infinite or NaN operand are NaN: in dK/dV
+  // a key or value of the sequence, in dQ's bias gradient a bias at an offset
+  // that no pair of the sequence has.
   int rows = INT_MAX;
 };
 __device__ __forceinline__ MaskCtx mask_make(int L, const int32_t* num_targets, int b, int max_attn_len, int ctx) {

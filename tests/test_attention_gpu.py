@@ -204,6 +204,37 @@ def test_generic_mask_bias_past_the_sequence(hip_lib, win, ctx, nts, D):
             assert bool(torch.isfinite(a).all()) and torch.equal(a, b), name
 
 
+@pytest.mark.parametrize("what", ["k", "v"])
+@pytest.mark.parametrize("win,ctx,nts,L,dtype", [(0, 0, [3], 300, "bf16"), (0, 0, [0], 129, "fp8"), (400, 0, None, 161, "bf16"),
+                                                 (0, 5, None, 385, "bf16"), (64, 3, [2], 97, "fp8")])
+def test_generic_mask_nonfinite_key(hip_lib, what, win, ctx, nts, L, dtype):
+    """An infinite key (or value) in the last tile of a sequence: its dV (dK)
+    is infinite, as the sum over the sequence's own rows gives it, and not NaN
+    from the rows past the sequence; the rows of the other keys are finite."""
+    ops = _ops()
+    at, D = L - 8, 128
+    g = torch.Generator().manual_seed(L)
+    q, k, v, dout = (torch.rand(L, 1, D, generator=g).to(torch.bfloat16) + 0.1 for _ in range(4))
+    scales = [None] * 3
+    if dtype == "fp8":
+        q, k, v = (t.to(torch.float8_e4m3fn) for t in (q, k, v))
+        scales = [torch.ones(L, 1, device=DEV) for _ in range(3)]
+        scales[1 if what == "k" else 2][at] = float("inf")
+    else:
+        (k if what == "k" else v)[at] = float("inf")
+    nt = None if nts is None else torch.tensor(nts, dtype=torch.int64, device=DEV)
+    grads = [torch.full((L, 1, D), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(3)]
+    ops.triton_hstu_attention_bwd(dout.to(DEV), q.to(DEV), k.to(DEV), v.to(DEV), *grads,
+                                  torch.tensor([0, L], device=DEV), nt, L, 0.1, win, ctx, None, False, 0, *scales,
+                                  full_fp8=False)
+    torch.cuda.synchronize()
+    # silu(inf) = inf and silu'(0 < x < inf) > 0 times an infinite dP, all terms of one sign
+    got = grads[2 if what == "k" else 1].cpu()
+    assert bool((got[at] == float("inf")).all())
+    other = torch.arange(L) != at
+    assert bool(torch.isfinite(got[other]).all())
+
+
 def test_strided_uvqk_views(hip_lib):
     """q/k/v read in place as column slices of a fused [T, 2048] buffer, and
     dq/dk/dv written into strided views of a fused gradient buffer."""
