@@ -209,14 +209,16 @@ __device__ __forceinline__ float sig_of_t(float t) {
 
 // Exponent argument t = -x*log2(e) of a score: raw MFMA dot product s times
 // the row factor c1 (-alpha*log2(e), times one operand's e4m3 scale) and the
-// other operand's scale c2 (e4m3 only), plus the pre-scaled bias b.
+// other operand's scale c2 (e4m3 only), plus the pre-scaled bias b.  The bias
+// is added in an explicit fused multiply-add: left to the compiler, some copies
+// of an epilogue round the product first, and a pair's score would depend on
+// the block form that its batch takes.
 template <bool FP8, bool BIAS>
 __device__ __forceinline__ float scaled_score(float s, float c1, float c2, float b) {
-  const float a = s * c1;
-  if constexpr (FP8 && BIAS) return __builtin_fmaf(a, c2, b);
-  else if constexpr (FP8) return a * c2;
-  else if constexpr (BIAS) return a + b;
-  else return a;
+  if constexpr (FP8 && BIAS) return __builtin_fmaf(s * c1, c2, b);
+  else if constexpr (FP8) return s * c1 * c2;
+  else if constexpr (BIAS) return __builtin_fmaf(s, c1, b);
+  else return s * c1;
 }
 
 // silu'(x) in terms of sg = sigmoid(x) and p = t * sg, where t = -x*log2(e):

@@ -742,3 +742,19 @@ def test_direct_grid_same_bytes(hip_lib, kind, D, H):
     for name, a, b in zip(("out", "dq", "dk", "dv"), *res):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), name
         assert bool((a.cpu()[pos >= N] == 0).all()) and not bool(torch.isnan(a).any()), name
+
+
+@pytest.mark.parametrize("far", ["const", "random"])
+@pytest.mark.parametrize("D,win,ctx", [(128, 0, 0), (64, 0, 0), (128, 0, 6)])
+def test_direct_grid_same_bytes_past_the_bias_range(hip_lib, far, D, win, ctx):
+    """Sequences well past the bias range (whole tiles of one bias value beside
+    tiles that look it up): the 64-query forward of a few sequences gives the
+    bytes of the 128-query one that the same sequences take among many."""
+    ops = _ops()
+    H, N, lengths = 4, 1024, [900, 517, 321, 1024, 130, 760]
+    q, k, v, _ = (t.to(DEV) for t in _case(lengths, H, D, seed=D + ctx))
+    bias = torch.full((H, 511), 0.25, device=DEV) if far == "const" else orc.make_bias(H, 256, seed=2, std=0.3).to(DEV)
+    outs = [ops.triton_hstu_attention_fwd(N, 0.1, q, k, v, orc.offsets_from_lengths(lengths + [0] * more).to(DEV), None,
+                                          win, ctx, None, False, 0, attn_bias=bias) for more in (0, 400)]
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
