@@ -291,7 +291,7 @@ __host__ __device__ inline int sched_items_of(int items, int x) {
 struct SeqCtx {
   int64_t start;
   int L, b, h, blk;
-  int tail;  // direct grid, first block of an item: rows past N that the item's outputs must zero
+  int tail;  // direct grid: rows past N, which the item's blocks zero (then it has all ceil(N / ROWS) of them)
 };
 // Workgroup -> (sequence, head, 128-row block).  heavy_last: the block with the
 // most key tiles is the last one of its sequence (forward, dQ) rather than the
@@ -342,7 +342,7 @@ __device__ __forceinline__ bool seq_ctx(const AttnParams& p, bool heavy_last, Se
   c.L = min((int)len, p.N);
   const int nb = (c.L + ROWS - 1) / ROWS;
   c.blk = heavy_last ? nb - 1 - m : m;
-  c.tail = p.sched_items == nullptr && m == 0 ? (int)len - c.L : 0;
+  c.tail = p.sched_items == nullptr ? (int)len - c.L : 0;
   return m < nb;
 }
 // Query blocks come last (the most keys) to first; with a contextual prefix the
@@ -351,11 +351,29 @@ template <int ROWS>
 __device__ __forceinline__ void prefix_block_first(const AttnParams& p, SeqCtx& c) {
   if (p.contextual_seq_len > 0) c.blk = c.blk == (c.L + ROWS - 1) / ROWS - 1 ? 0 : c.blk + 1;
 }
-// Zeroes columns h D .. h D + D - 1 of rows N .. N + tail - 1 of a sequence's
-// output (the set-up launch does it when there is a schedule).
-template <int D>
+// Zeroes columns h D .. h D + D - 1 of this block's share of rows N .. N +
+// tail - 1 of a sequence's output, every nb-th row (the set-up launch does it
+// when there is a schedule).  16-byte stores where the rows allow them.  It
+// stands before a block's work, where no register is taken yet: after it, the
+// accumulators were live and the full-FP8 dK/dV kernel spilled eight more.
+// Measured against an item's first block writing all of them, two bytes a
+// thread (us, bf16 forward, backward; H = 4, D = 128): 8 sequences of 2 048 cut
+// at 1 024 51.5 -> 26.9, 176 -> 79; 4 of 20 000 cut at 128 526 -> 28, 1 949 -> 126
+// (the set-up launch's four blocks a sequence: 86, 147; 1 046, 1 075).
+template <int D, int ROWS = 128>
 __device__ __forceinline__ void zero_tail(const SeqCtx& c, int N, uint16_t* out, int64_t rs) {
-  for (int i = threadIdx.x; i < c.tail * D; i += blockDim.x) out[(c.start + N + i / D) * rs + (int64_t)c.h * D + i % D] = 0;
+  const int nb = (N + ROWS - 1) / ROWS;
+  const int64_t end = (int64_t)N + c.tail;
+  uint16_t* o = out + c.start * rs + (int64_t)c.h * D;
+  if ((((uintptr_t)out | ((uint64_t)rs * 2)) & 15) == 0) {
+    constexpr int LPR = D / 8;
+    const int lr = threadIdx.x / LPR, col = threadIdx.x % LPR * 8, rpb = blockDim.x / LPR;
+    for (int64_t r = (int64_t)N + c.blk + (int64_t)nb * lr; r < end; r += (int64_t)nb * rpb)
+      *(u32x4*)(o + r * rs + col) = u32x4{0u, 0u, 0u, 0u};
+  } else {
+    const int lr = threadIdx.x / D, col = threadIdx.x % D, rpb = blockDim.x / D;
+    for (int64_t r = (int64_t)N + c.blk + (int64_t)nb * lr; r < end; r += (int64_t)nb * rpb) o[r * rs + col] = 0;
+  }
 }
 // dS tiles.  For the causal mask the dK/dV kernel computes dS for key block
 // kb (128 keys) against query tiles qt = 4 kb .. ceil(L/32) - 1 (32 queries);
@@ -455,7 +473,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
 
   SeqCtx sc;
   if (!seq_ctx<C::BM>(p, /*heavy_last=*/true, sc)) return;
-  if (sc.tail > 0) zero_tail<D>(sc, p.N, p.out, p.o_rs);
+  if (sc.tail > 0) zero_tail<D, C::BM>(sc, p.N, p.out, p.o_rs);
   const int L = sc.L, h = sc.h;
   if constexpr (GENERIC) prefix_block_first<C::BM>(p, sc);
   const int m0 = sc.blk * C::BM;
@@ -2392,9 +2410,9 @@ __global__ void __launch_bounds__(F8Bwd::NT, 3) hstu_bwd_f8_dkdv_kernel(AttnPara
   SeqCtx sc;
   int half = 0;
   if (!seq_ctx(p, /*heavy_last=*/false, sc, &half)) return;
-  if (sc.tail > 0 && half == 0) {
-    zero_tail<128>(sc, p.N, p.dk, p.dk_rs);
-    zero_tail<128>(sc, p.N, p.dv, p.dv_rs);
+  if (sc.tail > 0) {
+    if (half == 0) zero_tail<128>(sc, p.N, p.dk, p.dk_rs);
+    else zero_tail<128>(sc, p.N, p.dv, p.dv_rs);
   }
   const int L = sc.L, h = sc.h;
   const int n0 = sc.blk * C::BN;

@@ -758,3 +758,58 @@ def test_direct_grid_same_bytes_past_the_bias_range(hip_lib, far, D, win, ctx):
                                           win, ctx, None, False, 0, attn_bias=bias) for more in (0, 400)]
     torch.cuda.synchronize()
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("kind,D,mask", [("bf16", 128, 0), ("bf16", 64, 0), ("bf16", 128, 2), ("e4m3", 128, 0),
+                                         ("e4m3", 128, 2), ("full", 128, 0)])
+@pytest.mark.parametrize("pad", [0, 4])
+@pytest.mark.parametrize("N", [64, 300])
+def test_direct_grid_long_tails(hip_lib, kind, D, mask, pad, N):
+    """Rows past max_seq_len N, many times N of them, on a direct grid (each of
+    an item's blocks zeroes its share): zero in out, dq, dk and dv, and nothing
+    beside them; gradients as views of wider buffers, 16-byte aligned or not."""
+    ops = _ops()
+    H, lengths = 2, [N + 1, 3, N, 5 * N + 77, 0, 2 * N + 130]
+    q, k, v, offs = _case(lengths, H, D, seed=N)
+    T = q.shape[0]
+    q, k, v, dout = (t.to(DEV) for t in (q, k, v, q.flip(0)))
+    scales = [None] * 3
+    if kind != "bf16":
+        q, k, v = ((t.float() * 100).to(torch.float8_e4m3fn) for t in (q, k, v))
+        scales = [torch.full((T, H), 0.01, device=DEV) for _ in range(3)]
+    full = kind == "full"
+    out = ops.triton_hstu_attention_fwd(N, 0.1, q, k, v, offs.to(DEV), None, 0, mask, None, False, 0, *scales,
+                                        fp8_pv=full)
+    wide = [torch.full((T, H * D + pad), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(3)]
+    grads = [w[:, :H * D].view(T, H, D) if pad == 0 else w[:, :H * D].unflatten(1, (H, D)) for w in wide]
+    ops.triton_hstu_attention_bwd(dout, q, k, v, *grads, offs.to(DEV), None, N, 0.1, 0, mask, None, False, 0, *scales,
+                                  full_fp8=full)
+    torch.cuda.synchronize()
+    pos = torch.cat([torch.arange(n) for n in lengths])
+    for name, a in zip(("out", "dq", "dk", "dv"), (out, *grads)):
+        a = a.cpu()
+        assert bool((a[pos >= N] == 0).all()), name
+        assert bool(torch.isfinite(a).all()) and bool((a[pos < N] != 0).any()), name
+    if pad:
+        assert all(bool(torch.isnan(w[:, H * D:]).all()) for w in wide)
+
+
+def test_direct_grid_tail_past_2_31_elements(hip_lib):
+    """A sequence with more than 2^31 elements of a head past max_seq_len: all
+    of them are zeroed."""
+    from hstu_amd import _lib
+
+    N, D = 64, 128
+    T = N + 2 ** 24 + 5
+    q = torch.zeros(T, 1, D, dtype=torch.bfloat16, device=DEV)
+    q[:N] = 0.5
+    out = torch.full((T, D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    offs = torch.tensor([0, T], device=DEV)
+    ws = torch.empty(_lib.fn("hstu_attn_fwd_workspace_bytes")(0, T, 1, 1, D, N), dtype=torch.uint8, device=DEV)
+    st = _lib.fn("hstu_attn_fwd")(0, q.data_ptr(), q.data_ptr(), q.data_ptr(), D, D, D, None, None, None, 0, 0,
+                                  offs.data_ptr(), 1, 1, D, N, 0.1, None, 0, 0, None, 0, out.data_ptr(), D,
+                                  ws.data_ptr(), ws.numel(), T, torch.cuda.current_stream().cuda_stream)
+    _lib.check(st, "hstu_attn_fwd")
+    torch.cuda.synchronize()
+    assert int(torch.count_nonzero(out[N:].view(torch.int16))) == 0
+    assert bool((out[:N] > 0).all())
