@@ -317,19 +317,22 @@ __device__ __forceinline__ bool seq_ctx(const AttnParams& p, bool heavy_last, Se
     // the last of the XCD's n items whose first block is <= k: the lanes look at
     // 64 of them at once, two dependent loads where a binary search had log2 n
     // (the masked training batch above, 1 200 short blocks in three kernels:
-    // 242.6 -> 239.2 us)
+    // 242.6 -> 239.2 us); among more, a binary search over scalar loads first
+    // brings them down to 64
     const int lane = threadIdx.x & 63, n = sched_items_of(p.B * p.H, x);
     const int* st = p.sched_start + x * (p.sched_cap + 1);
     const int total = st[n];
-    int base = 0;
-    for (int c0 = 0; n > 64 && c0 < n; c0 += 64 * 64) {  // the chunk of 64 items
-      const int c = c0 + 64 * lane;
-      const int le = __popcll(__ballot((c < n ? st[c] : INT_MAX) <= k));
-      if (le > 0) base = c0 + 64 * (le - 1);
-      if (le < 64) break;
+    int lo = 0, hi = n;
+    if (n > 64) {
+      if (k >= total) return false;
+      while (hi - lo > 64) {
+        const int mid = (lo + hi) >> 1;
+        if (st[mid] <= k) lo = mid;
+        else hi = mid;
+      }
     }
-    const int j = base + lane;
-    const int first = j < n ? st[j] : INT_MAX, item = j < n ? p.sched_items[x * p.sched_cap + j] : 0;
+    const int j = lo + lane;
+    const int first = j < hi ? st[j] : INT_MAX, item = j < hi ? p.sched_items[x * p.sched_cap + j] : 0;
     if (k >= total) return false;
     const int at = __popcll(__ballot(first <= k)) - 1;
     bh = __builtin_amdgcn_readlane(item, at);
@@ -3078,12 +3081,22 @@ __device__ void schedule_block(const int64_t* seq_offsets, int B, int H, int N, 
   for (int b = tid; b < B; b += kSchedBins) rank[b] = atomicAdd(&bins[min(nbv[b], kSchedBins - 1)], 1);
   __syncthreads();
   // item r = rank*H + head -> XCD by snake order, dense index j on that XCD
-  for (int i = tid; i < B * H; i += kSchedBins) {
-    const int b = i / H, r = rank[b] * H + (i - b * H), q = r & 15;
-    const int x = q < 8 ? q : 15 - q;
+  auto place = [&](int i, int r, int nb) {
+    const int q = r & 15, x = q < 8 ? q : 15 - q;
     const int j = (r >> 4) * 2 + (q >= 8 ? 1 : 0);
     items[x * cap + j] = i;
-    cnt[x * (cap + 1) + j] = nbv[b];
+    cnt[x * (cap + 1) + j] = nb;
+  };
+  if (B < kSchedBins) {  // an item a thread
+    for (int i = tid; i < B * H; i += kSchedBins) {
+      const int b = i / H;
+      place(i, rank[b] * H + (i - b * H), nbv[b]);
+    }
+  } else {  // a sequence a thread: rank and count (in memory now) are read once, not per head
+    for (int b = tid; b < B; b += kSchedBins) {
+      const int nb = nbv[b], r = rank[b] * H;
+      for (int h = 0; h < H; ++h) place(b * H + h, r + h, nb);
+    }
   }
   __syncthreads();
   // per XCD (one wave each): exclusive scan of the block counts

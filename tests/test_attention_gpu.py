@@ -813,3 +813,44 @@ def test_direct_grid_tail_past_2_31_elements(hip_lib):
     torch.cuda.synchronize()
     assert int(torch.count_nonzero(out[N:].view(torch.int16))) == 0
     assert bool((out[:N] > 0).all())
+
+
+@pytest.mark.parametrize("B,H,N,kind", [(700, 1, 300, "bf16"), (700, 4, 40, "full"), (1023, 2, 40, "bf16"),
+                                        (1024, 2, 40, "targets"), (9000, 4, 24, "bf16"), (9000, 4, 24, "full")])
+def test_many_sequences_same_bytes(hip_lib, B, H, N, kind):
+    """Batches on both sides of the schedule's sizes (64 and 1 024 sequences or
+    items, 4 096 items an XCD): out, dq, dk and dv are the bytes of the same
+    sequences in batches small enough for a direct grid."""
+    ops = _ops()
+    D = 128 if kind == "full" else 64
+    g = torch.Generator().manual_seed(B + H)
+    lengths = torch.randint(0, N + 1, (B,), generator=g)
+    T = int(lengths.sum())
+    q, k, v, dout = (torch.randn(T, H, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(4))
+    nt = torch.minimum(lengths, torch.randint(0, 5, (B,), generator=g)).to(DEV) if kind == "targets" else None
+    scales = [None] * 3
+    if kind == "full":
+        q, k, v = ((t.float() * 50).to(torch.float8_e4m3fn) for t in (q, k, v))
+        scales = [torch.full((1,), 0.02, device=DEV) for _ in range(3)]
+
+    def run(b0, b1):
+        off = orc.offsets_from_lengths(lengths[b0:b1].tolist()).to(DEV)
+        t0, t1 = int(lengths[:b0].sum()), int(lengths[:b1].sum())
+        qs, ks, vs, do = (t[t0:t1] for t in (q, k, v, dout))
+        tgt = None if nt is None else nt[b0:b1]
+        out = ops.triton_hstu_attention_fwd(N, 0.1, qs, ks, vs, off, tgt, 0, 0, None, False, 0, *scales,
+                                            fp8_pv=kind == "full")
+        grads = [torch.full(qs.shape, float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(3)]
+        ops.triton_hstu_attention_bwd(do, qs, ks, vs, *grads, off, tgt, N, 0.1, 0, 0, None, False, 0, *scales,
+                                      full_fp8=kind == "full")
+        return [out, *grads]
+
+    step = (15 if kind == "full" else 1280) // (H * ((N + 127) // 128))  # direct for the full-FP8 backward: under 16 items
+    step = max(step, B // 40) if kind == "full" else step
+    whole = run(0, B)
+    parts = [run(b, min(b + step, B)) for b in range(0, B, step)]
+    torch.cuda.synchronize()
+    for i, name in enumerate(("out", "dq", "dk", "dv")):
+        got = torch.cat([p[i] for p in parts])
+        assert bool(torch.isfinite(got).all()), name
+        assert torch.equal(whole[i].view(torch.int16), got.view(torch.int16)), name
