@@ -1809,6 +1809,8 @@ hipError_t set_gemm_lds(const void* fn) {
 // (256) 22.8 / 15.4, 12.0 / 10.7.
 constexpr int kFewMaxWideTiles = 80;
 bool few_rows(int M, int N) { return (int64_t)((M + kBM - 1) / kBM) * (N / kWideBN) <= kFewMaxWideTiles; }
+// 128 x 128 tiles that the tile kernel runs in one round, one a CU.
+constexpr int kTileRound = 256;
 int launch_few_rows(void (*kern)(GemmParams), GemmParams p, hipStream_t stream) {
   p.tiles_m = (p.M + kFewB - 1) / kFewB;
   p.tiles_n = p.N / kFewB;
@@ -1956,19 +1958,32 @@ extern "C" int hstu_bf16_gemm(const void* A, int64_t lda, const void* W, int64_t
   p.silu_begin = silu_begin;
   p.silu_end = silu_end;
   p.tiles_m = (M + kBM - 1) / kBM;
-  // two-workgroup form (few rows: the few-row form, the same MFMA chain):
   // whole 256-column tiles, at least two k-steps, 16-byte output and residual
-  // rows, a SiLU range of whole waves (64 columns).  duo_ok does not look at M,
-  // so a row's bytes do not depend on its batch.
+  // rows, a SiLU range of whole waves (64 columns): few rows take the few-row
+  // form, products of more 128 x 128 tiles than CUs the two-workgroup form, and
+  // those between the tile kernel below, one tile a CU where the two-workgroup
+  // form would leave half of the CUs idle.  Measured (us, two-workgroup / tile):
+  // [8 000, 2048] x [2048, 512] (252 tiles) 33.1 / 29.0, [5 120, 512] x [512, 512]
+  // (160) 11.4 / 10.6, [16 000, 512] x [512, 256] (250) 13.4 / 11.4, [2 100, 512] x
+  // [512, 1536] (204) 13.2 / 11.2; [2 100, 512] x [512, 2048] (272) 13.6 / 15.5,
+  // [12 000, 2048] x [2048, 512] (376) 37.2 / 41.9.  A row's bytes do not depend
+  // on its batch: the three forms sum over k in the same order, and a 16x16x32
+  // MFMA rounds as two 32x32x16 ones (no byte differs, cancelling sums included).
   const bool duo_ok = N % kWideBN == 0 && p.K >= 2 * kBK && (uintptr_t)C % 16 == 0 && ldc % 8 == 0 &&
                       (!residual || ((uintptr_t)residual % 16 == 0 && ldr % 8 == 0)) &&
                       (silu_begin >= silu_end || (silu_begin % 64 == 0 && silu_end % 64 == 0)) &&
                       (int64_t)kBM * 2 * ldc <= 0xffffffffLL && (int64_t)kBM * 2 * ldr <= 0xffffffffLL &&
                       (int64_t)(kWideBN - 1) * p.ldw + p.K <= 0xffffffffLL;
-  if (duo_ok && few_rows(M, N))
+  // With few columns (N <= 512) a second round of few-row tiles
+  // costs more than the tile kernel from K = 512 on (us, few-row / tile: [4 900,
+  // 2048] x [2048, 512] 29.1 / 26.9, [4 900, 512] 11.0 / 10.3; [4 900, 256] 6.9 /
+  // 7.8, [1 280, 2048] x [2048, 2048] 24.5 / 28.4); a few tiles more than the 512
+  // slots do not ([4 100, 512], 520 tiles, 9.7 / 10.1).
+  const bool second_round = N <= 512 && K >= 512 && (int64_t)((M + kFewB - 1) / kFewB) * (N / kFewB) > 528;
+  if (duo_ok && few_rows(M, N) && !second_round)
     return launch_few_rows(residual ? gemm_few_rows_kernel<false, true, kBF16> : gemm_few_rows_kernel<false, false, kBF16>,
                            p, stream);
-  if (duo_ok) {
+  if (duo_ok && (int64_t)p.tiles_m * (N / kBN) > kTileRound) {
     p.tiles_n = N / kWideBN;
     int per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
     void* args[] = {&p, &per_xcd};

@@ -367,3 +367,33 @@ def test_gemm_few_row_form_same_bytes(hip_lib, fmt, N, K, resid, out8):
     for rows in (1, 64, 65, 300):
         s = slice(200, 200 + rows)
         assert torch.equal(full[s], run(s).view(torch.uint8)), rows
+
+
+@pytest.mark.parametrize("N,K,resid", [(256, 128, False), (512, 2048, False), (512, 1536, True), (768, 192, True)])
+@pytest.mark.parametrize("kind", ["randn", "cancel"])
+def test_bf16_gemm_forms_same_bytes(hip_lib, N, K, resid, kind):
+    """The three bf16 forms give a row the same bytes: a product of 128 x 128
+    tiles for more than one round of the chip (two-workgroup form), its rows in
+    batches of at most one round (tile kernel) and of a few tiles (few-row
+    form), and all of it with 8-byte aligned output rows (tile kernel).
+    ``cancel``: sums that cancel, so that the result is their rounding."""
+    fp8 = _fp8()
+    g = torch.Generator().manual_seed(N + K)
+    M = 128 * (256 * 128 // N + 2) + 9
+    a = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16)
+    if kind == "cancel":
+        perm = torch.randperm(K // 2, generator=g)
+        a[:, K // 2:] = a[:, :K // 2][:, perm]
+        w[:, K // 2:] = -w[:, :K // 2][:, perm]
+    a, w = a.to(DEV), w.to(DEV)
+    b = None if kind == "cancel" else (0.1 * torch.randn(N, generator=g)).to(torch.bfloat16).to(DEV)
+    r = torch.randn(M, N, generator=g).to(torch.bfloat16).to(DEV) if resid and kind != "cancel" else None
+    run = lambda x, y, out=None: fp8.bf16_gemm(x, w, bias=b, residual=y, silu_cols=(64, 128), out=out)  # noqa: E731
+    full = run(a, r).view(torch.int16)
+    for step in (128 * (128 * 256 // N) - 7, 128 * (60 * 256 // N)):  # at most 256 tiles; 60 wide ones
+        got = torch.cat([run(a[i:i + step], None if r is None else r[i:i + step]) for i in range(0, M, step)])
+        assert torch.equal(full, got.view(torch.int16)), step
+    wide = torch.empty(M, N + 4, dtype=torch.bfloat16, device=DEV)
+    run(a, r, out=wide[:, :N])
+    assert torch.equal(full, wide[:, :N].contiguous().view(torch.int16))
