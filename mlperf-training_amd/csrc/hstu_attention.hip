@@ -43,6 +43,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <climits>
 #include <mutex>
 #include <type_traits>
@@ -3407,7 +3408,7 @@ int fwd_launch(int dtype, const void* q, const void* k, const void* v, int64_t q
                int64_t scale_row_stride, int64_t scale_head_stride, const int64_t* seq_offsets, int B, int H, int D,
                int max_seq_len, float alpha, const int32_t* num_targets, int max_attn_len, int contextual_seq_len,
                const float* attn_bias, int bias_R, void* out, int64_t out_row_stride, int* sched_ws,
-               hipStream_t stream, float pv_scale = 0.f) {
+               int64_t total_tokens, hipStream_t stream, float pv_scale = 0.f) {
   AttnParams p{};
   p.q = (const uint8_t*)q;
   p.k = (const uint8_t*)k;
@@ -3436,11 +3437,14 @@ int fwd_launch(int dtype, const void* q, const void* k, const void* v, int64_t q
   const bool direct = direct_grid(B, H, max_seq_len, /*prep=*/false);
   const int grid = sched_grid(B, H, max_seq_len, direct);
   // 64-query blocks (bf16) while the 128-query ones are at most 512, one round
-  // of the chip.  Measured (us, 128 / 64; H = 4, D = 128): one sequence of 3 001
-  // (96 blocks) 71.0 / 50.8, D = 64 47.6 / 34.2; 16 of up to 1024 (512)
-  // 31.7 / 26.0; 8 of up to 2048 (512) 49.8 / 40.2; 32 of up to 1024 (1024)
-  // 38.2 / 41.2.
-  const bool half = direct && grid <= 512 && dtype == HSTU_DTYPE_BF16;
+  // of the chip; the grid's slots bound their number and so do the tokens, which
+  // count where a few sequences are much longer than the others.  Measured (us,
+  // 128 / 64; H = 4, D = 128): one sequence of 3 001 (96 blocks) 71.0 / 50.8, D = 64
+  // 47.6 / 34.2; 16 of up to 1024 (512) 31.7 / 26.0; 8 of up to 2048 (512)
+  // 49.8 / 40.2; 32 of up to 1024 (1024) 38.2 / 41.2; one of 4 096 and nine of 40
+  // (1 280 slots, at most 176 blocks) 106.1 / 81.0, with targets 109.8 / 83.3.
+  const int64_t blocks = std::min<int64_t>(grid, H * (total_tokens / 128 + B));
+  const bool half = direct && blocks <= 512 && dtype == HSTU_DTYPE_BF16;
   p.bias = attn_bias;
   p.bias_R = bias_R;
   // the block schedule, and the rows past max_seq_len zeroed, in one launch
@@ -3505,7 +3509,7 @@ extern "C" int hstu_attn_fwd(int dtype, const void* q, const void* k, const void
   return fwd_launch(dtype, q, k, v, q_row_stride, k_row_stride, v_row_stride, q_scale, k_scale, v_scale,
                     scale_row_stride, scale_head_stride, seq_offsets, B, H, D, max_seq_len, alpha, num_targets,
                     max_attn_len, contextual_seq_len, attn_bias, bias_R, out, out_row_stride, (int*)workspace,
-                    stream);
+                    total_tokens, stream);
 }
 
 extern "C" int hstu_attn_fwd_fp8_pv_max_seq_len(void) {
@@ -3535,7 +3539,8 @@ extern "C" int hstu_attn_fwd_fp8_pv(const void* q, const void* k, const void* v,
   if (workspace == nullptr || workspace_bytes < fwd_workspace_bytes(B, H)) return HSTU_E_BAD_ARG;
   return fwd_launch(HSTU_DTYPE_FP8_E4M3, q, k, v, q_row_stride, k_row_stride, v_row_stride, q_scale, k_scale,
                     v_scale, scale_row_stride, scale_head_stride, seq_offsets, B, H, D, max_seq_len, alpha, nullptr, 0,
-                    0, attn_bias, bias_R, out, out_row_stride, (int*)workspace, stream, pv_scale);
+                    0, attn_bias, bias_R, out, out_row_stride, (int*)workspace, total_tokens, stream,
+                    pv_scale);
 }
 
 // ---------------------------------------------------------------------------
@@ -3593,7 +3598,8 @@ extern "C" int hstu_attn_fwd_noalloc(int dtype, const void* q, const void* k, co
   if (e != hipSuccess) return (int)e;
   return fwd_launch(dtype, q, k, v, q_row_stride, k_row_stride, v_row_stride, q_scale, k_scale, v_scale,
                     scale_row_stride, scale_head_stride, seq_offsets, B, H, D, max_seq_len, alpha, num_targets,
-                    max_attn_len, contextual_seq_len, attn_bias, bias_R, out, out_row_stride, (int*)ws, stream);
+                    max_attn_len, contextual_seq_len, attn_bias, bias_R, out, out_row_stride, (int*)ws, total_tokens,
+                    stream);
 }
 
 namespace {

@@ -854,3 +854,21 @@ def test_many_sequences_same_bytes(hip_lib, B, H, N, kind):
         got = torch.cat([p[i] for p in parts])
         assert bool(torch.isfinite(got).all()), name
         assert torch.equal(whole[i].view(torch.int16), got.view(torch.int16)), name
+
+
+@pytest.mark.parametrize("kind", ["causal", "bias", "targets"])
+def test_skewed_batch_same_bytes(hip_lib, kind):
+    """One long sequence among short ones: a grid of more than 512 block slots
+    but few blocks takes the 64-query forward; the bytes are those of the
+    128-query one that the same sequences take among many."""
+    ops = _ops()
+    H, D, N, lengths = 4, 128, 2048, [20] * 9 + [1999] + [37] * 10
+    q, k, v, _ = (t.to(DEV) for t in _case(lengths, H, D, seed=3))
+    bias = orc.make_bias(H, 128, seed=2, std=0.3).to(DEV) if kind == "bias" else None
+    outs = []
+    for more in (0, 400):
+        nt = torch.tensor([5] * len(lengths) + [0] * more, device=DEV) if kind == "targets" else None
+        outs.append(ops.triton_hstu_attention_fwd(N, 0.1, q, k, v, orc.offsets_from_lengths(lengths + [0] * more).to(DEV),
+                                                  nt, 0, 0, None, False, 0, attn_bias=bias))
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
