@@ -179,6 +179,53 @@ def test_generic_mask_tiles(hip_lib, win, ctx, nts, D, with_bias):
         assert orc.rel_l2(db, bd.grad.double().cpu()) <= 1e-2
 
 
+@pytest.mark.parametrize("form", ["direct", "scheduled"])
+@pytest.mark.parametrize("dtype,win,ctx,nts,D,with_bias", [
+    ("bf16", 63, 0, None, 128, False), ("bf16", 65, 33, None, 64, True), ("bf16", 200, 130, [7, 64, 3, 1], 128, True),
+    ("bf16", 0, 129, [200, 0, 2, 1], 64, False), ("bf16", 0, 0, [130, 65, 255, 1], 128, True),
+    ("e4m3", 1, 0, None, 128, False), ("e4m3", 64, 0, [0, 64, 255, 1], 128, True), ("e4m3", 31, 2, [1, 128, 33, 2], 128, False),
+    ("e4m3", 0, 129, None, 128, True), ("e4m3", 200, 130, [7, 64, 3, 1], 128, True)])
+def test_generic_mask_tiles_large_grids(hip_lib, form, dtype, win, ctx, nts, D, with_bias):
+    """The masks of test_generic_mask_tiles in the 128-query forms, in bf16 and
+    e4m3: enough empty sequences follow for a direct grid of more than 512
+    blocks (N = 256), or for the scheduled grid (N = 400).  Forward, dq, dk, dv
+    and the bias gradient against the float64 oracle on the rounded inputs, at
+    the bf16 bar (bf16) and at 1.5e-2 relative L2 (e4m3)."""
+    ops = _ops()
+    lengths, N, H, empty = ([256, 129, 255, 3], 256, 2, 296) if form == "direct" else ([385, 129, 257, 3], 400, 2, 300)
+    q, k, v, offs = _case(lengths, H, D, seed=win + ctx)
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
+    ntt = None if nts is None else torch.tensor([min(a, b) for a, b in zip(nts, lengths)], dtype=torch.int64)
+    bias = orc.make_bias(H, 100, seed=2, std=0.3) if with_bias else None
+    alpha, scales, ref_in = 0.15, [None] * 3, (q, k, v)
+    if dtype == "e4m3":
+        packed = [_quantize(t.float()) for t in (q, k, v)]
+        ref_in = [orc.dequantize(*p) for p in packed]
+        q, k, v = (p[0] for p in packed)
+        scales = [p[1].contiguous().to(DEV) for p in packed]
+    od = orc.offsets_from_lengths(lengths + [0] * empty).to(DEV)
+    ntd = None if ntt is None else torch.cat([ntt, torch.zeros(empty, dtype=torch.int64)]).to(DEV)
+    qd, kd, vd = (t.to(DEV) for t in (q, k, v))
+    bd = None if bias is None else bias.to(DEV)
+    db = None if bias is None else torch.full_like(bd, float("nan"))
+    out = ops.triton_hstu_attention_fwd(N, alpha, qd, kd, vd, od, ntd, win, ctx, None, False, 0, *scales, attn_bias=bd)
+    grads = [torch.full(dout.shape, float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(3)]
+    ops.triton_hstu_attention_bwd(dout.to(DEV), qd, kd, vd, *grads, od, ntd, N, alpha, win, ctx, None, False, 0, *scales,
+                                  attn_bias=bd, dbias=db, full_fp8=False)
+    torch.cuda.synchronize()
+    ref = orc.hstu_mha_dense(N, alpha, *(t.double() for t in ref_in), offs, ntt, win, ctx,
+                             None if bias is None else bias.double(), dtype=torch.float64)
+    refs = orc.hstu_mha_bwd(N, alpha, *ref_in, offs, dout, ntt, win, ctx, bias)
+    for name, got, r in zip(("fwd", "dq", "dk", "dv"), (out, *grads), (ref, *refs[:3])):
+        got, s = got.float().cpu(), r.abs().max()
+        if dtype == "bf16":
+            _check_bf16(got / s, r / s, name)
+        else:
+            assert orc.rel_l2(r, got) <= 1.5e-2, name
+    if bias is not None:
+        assert orc.rel_l2(refs[3], db.double().cpu()) <= (1e-2 if dtype == "bf16" else 1.5e-2)
+
+
 @pytest.mark.parametrize("win,ctx,nts,D", [(0, 0, [0, 64], 64), (500, 0, None, 128), (0, 33, [7, 0], 128), (0, 2, None, 64)])
 def test_generic_mask_bias_past_the_sequence(hip_lib, win, ctx, nts, D):
     """A bias that is infinite or NaN at offsets that no pair has: the rows of

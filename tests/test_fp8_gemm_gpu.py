@@ -90,8 +90,10 @@ def test_gemm_residual_k1536(hip_lib):
     assert float((got - ref).abs().max() / ref.abs().max()) <= 1e-2
 
 
-def test_gemm_e4m3_out(hip_lib):
-    """VQK projection emitting e4m3 at an output scale (scaled_mm_fp8_out_preq).
+@pytest.mark.parametrize("M", [700, 128 * 14 + 5])
+def test_gemm_e4m3_out(hip_lib, M):
+    """VQK projection emitting e4m3 at an output scale (scaled_mm_fp8_out_preq),
+    in the few-row form (36 wide tiles) and the two-workgroup form (90).
 
     Bar: every element within one e4m3 half-step (2^-4 relative) of the
     float64 result / out_scale, plus 2.5e-5 * max|result| absolute.  The
@@ -99,7 +101,7 @@ def test_gemm_e4m3_out(hip_lib):
     about 7e-6 * max (the same deviation appears on the bf16 output path), so
     near-zero elements can land one e4m3 step from the float64 rounding."""
     fp8 = _fp8()
-    M, N, K = 700, 1536, 512
+    N, K = 1536, 512
     a8, sa, w8t, sw = _operands(M, N, K, seed=6, per_row=False, per_col=False)
     bias = (torch.randn(N, generator=torch.Generator().manual_seed(7)) * 0.1).to(torch.bfloat16)
     ref = orc.fp8_rowcol_gemm(a8, sa, w8t.t(), sw, bias=bias.float())
@@ -238,14 +240,17 @@ def test_gemm_k512_both_kernels(hip_lib):
 
 
 @pytest.mark.parametrize("out8", [False, True])
-def test_gemm_pc_kernel_bounds(hip_lib, out8):
-    """The producer/consumer kernel (N % 256, K % 256, 64-aligned SiLU) on a
-    ragged M with a padded row stride: every valid element against the
-    oracle, and nothing written past N in a row nor past row M (its stores
-    are bounded by buffer resources at the tile's valid rows)."""
+@pytest.mark.parametrize("M,N", [(777, 512), (128 * 41 + 9, 512), (128 * 81 + 1, 256), (128 * 27 + 77, 768)])
+def test_gemm_pc_kernel_bounds(hip_lib, M, N, out8):
+    """The wide forms (N % 256, K % 256, 64-aligned SiLU) on a ragged M with a
+    padded row stride: every valid element against the oracle, and nothing
+    written past N in a row nor past row M (the stores are bounded by buffer
+    resources at the tile's valid rows).  14 tiles of 128 x 256 run the few-row
+    kernel, 84 and 82 at N <= 512 the producer/consumer kernel, 84 at N = 768 the
+    two-workgroup kernel."""
     import hstu_amd._lib as lib
 
-    M, N, K = 777, 512, 1024
+    K = 1024
     a8, sa, w8t, sw = _operands(M, N, K, seed=31)
     bias = (torch.randn(N, generator=torch.Generator().manual_seed(32)) * 0.1).to(torch.bfloat16)
     ref = orc.fp8_rowcol_gemm(a8, sa, w8t.t(), sw, bias=bias.float(), silu_cols=(64, 192))
@@ -275,8 +280,8 @@ def test_gemm_pc_kernel_bounds(hip_lib, out8):
                                                    (257, 2048, 512, True, False, True),
                                                    (130, 512, 1536, False, True, False)])
 def test_bf16_gemm(hip_lib, M, N, K, bias, resid, silu):
-    """The bf16 mode of the tile kernel (``hstu_bf16_gemm``): against the
-    float64 product of the same bf16 operands with the same epilogue;
+    """``hstu_bf16_gemm`` (few-row form at these sizes): against the float64
+    product of the same bf16 operands with the same epilogue;
     relative L2 <= 4e-3, max |err| <= 1e-2 * max |ref| (bf16 output)."""
     fp8 = _fp8()
     g = torch.Generator().manual_seed(M + N + K)
@@ -301,10 +306,11 @@ def test_bf16_gemm(hip_lib, M, N, K, bias, resid, silu):
 
 def test_bf16_gemm_rows_independent_of_batch(hip_lib):
     """A row's result does not depend on the other rows of the batch: rows of
-    a 4096-row product equal the same rows computed in a 300-row batch."""
+    a 12 000-row product (two-workgroup form) equal the same rows computed in a
+    300-row batch (few-row form)."""
     fp8 = _fp8()
     g = torch.Generator().manual_seed(9)
-    a = torch.randn(4096, 2048, generator=g).to(torch.bfloat16).to(DEV)
+    a = torch.randn(12000, 2048, generator=g).to(torch.bfloat16).to(DEV)
     w = (torch.randn(512, 2048, generator=g) / 45).to(torch.bfloat16).to(DEV)
     full = fp8.bf16_gemm(a, w)
     part = fp8.bf16_gemm(a[1000:1300], w)
@@ -314,20 +320,26 @@ def test_bf16_gemm_rows_independent_of_batch(hip_lib):
 
 @pytest.mark.parametrize("M,N,K,resid,pad", [(1, 256, 128, True, 0), (127, 512, 192, False, 0), (129, 256, 320, True, 8),
                                              (385, 768, 128, False, 8), (200, 256, 64, False, 0),
-                                             (200, 256, 128, True, 4)])
+                                             (200, 256, 128, True, 4), (128 * 128 + 1, 256, 128, True, 8),
+                                             (128 * 129 + 77, 256, 192, False, 0), (128 * 128 + 65, 256, 320, True, 8),
+                                             (128 * 64 + 9, 512, 256, False, 8), (128 * 43 + 127, 768, 128, False, 8),
+                                             (128 * 100 + 3, 256, 192, True, 8), (128 * 128 + 1, 256, 64, False, 0)])
 def test_bf16_gemm_two_workgroup_form(hip_lib, M, N, K, resid, pad):
-    """The two-workgroup bf16 form at its edges: two and three k-steps, ragged
-    last row tiles, strided rows; one k-step and 8-byte aligned output rows
-    (``pad`` 4) take the tile kernel.  Against the float64 product: relative
-    L2 <= 4e-3 (one bf16 rounding of a fp32 sum is 1.7e-3), SiLU on the second
-    64 columns, columns outside the output untouched."""
+    """The bf16 forms at their edges: two, three and more k-steps, ragged last
+    row tiles, strided rows.  Up to 385 rows run the few-row form, 101 row tiles
+    at N = 256 the tile kernel, the others above 128 row tiles (64 at N = 512, 43
+    at N = 768) the two-workgroup form; one k-step and 8-byte aligned output rows
+    (``pad`` 4) take the tile kernel.  Against the float64 product: relative L2
+    <= 4e-3 (one bf16 rounding of a fp32 sum is 1.7e-3), SiLU on the second 64
+    columns, columns outside the output and rows past it untouched."""
     fp8 = _fp8()
     g = torch.Generator().manual_seed(M + N + K)
     a = torch.randn(M, K + 16, generator=g).to(torch.bfloat16)[:, 8:K + 8]
     w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16)
     b = (0.1 * torch.randn(N, generator=g)).to(torch.bfloat16)
     r = torch.randn(M, N, generator=g).to(torch.bfloat16) if resid else None
-    wide = torch.full((M, N + pad + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    past = torch.full((M + 130, N + pad + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    wide = past[:M]
     ad = torch.empty(M, K + 16, dtype=torch.bfloat16, device=DEV)[:, 8:K + 8]
     ad.copy_(a)
     fp8.bf16_gemm(ad, w.to(DEV), bias=b.to(DEV), residual=None if r is None else r.to(DEV), silu_cols=(64, 128),
@@ -337,18 +349,22 @@ def test_bf16_gemm_two_workgroup_form(hip_lib, M, N, K, resid, pad):
     if r is not None:
         ref = ref + r.double()
     assert orc.rel_l2(ref, wide[:, :N].cpu().double()) <= 4e-3
-    assert bool((wide[:, N:] == 7.0).all())
+    assert bool((wide[:, N:] == 7.0).all()) and bool((past[M:] == 7.0).all())
 
 
 @pytest.mark.parametrize("fmt,N,K,resid,out8", [("bf16", 512, 128, False, False), ("bf16", 512, 1536, True, False),
                                                 ("e4m3", 512, 1536, True, False), ("e4m3", 768, 256, False, True),
-                                                ("e4m3", 256, 512, True, True), ("e4m3", 2048, 512, False, False)])
+                                                ("e4m3", 256, 512, True, True), ("e4m3", 2048, 512, False, False),
+                                                ("e4m3", 512, 512, False, False), ("e4m3", 256, 1024, False, True),
+                                                ("e5m2", 512, 2048, False, False), ("e5m2", 1536, 512, False, False)])
 def test_gemm_few_row_form_same_bytes(hip_lib, fmt, N, K, resid, out8):
-    """The few-row form gives the bytes of the wide forms: 1, 64, 65 and 300
-    rows of a product large enough for the wide form, computed alone."""
+    """The few-row form gives the bytes of the forms that more rows take (bf16:
+    the tile kernel; fp8: the two-workgroup form, at N <= 512 without a residual
+    the producer/consumer form): 1, 64, 65 and 300 rows of such a product,
+    computed alone, and its last ragged rows."""
     fp8 = _fp8()
     g = torch.Generator().manual_seed(N + K)
-    M = 128 * (81 * 256 // N + 1)
+    M = 128 * (81 * 256 // N + 1) + 41
     a = torch.randn(M, K, generator=g).to(torch.bfloat16)
     w = torch.randn(N, K, generator=g) / K ** 0.5
     b = None if resid else (0.1 * torch.randn(N, generator=g)).to(torch.bfloat16).to(DEV)
@@ -356,6 +372,12 @@ def test_gemm_few_row_form_same_bytes(hip_lib, fmt, N, K, resid, out8):
     if fmt == "bf16":
         ad, wd = a.to(DEV), w.to(torch.bfloat16).to(DEV)
         run = lambda s: fp8.bf16_gemm(ad[s], wd, bias=b, residual=None if r is None else r[s])  # noqa: E731
+    elif fmt == "e5m2":
+        from hstu_amd import bwd_fp8
+
+        a8, w8 = (a * 8).to(torch.float8_e5m2).to(DEV), (w * 400).to(torch.float8_e4m3fn).to(DEV)
+        sg, sw = torch.tensor([0.02], device=DEV), torch.tensor([0.003], device=DEV)
+        run = lambda s: bwd_fp8.fp8_dgrad(a8[s], sg, w8, sw)  # noqa: E731
     else:
         a8, sa = fp8.quantize_e4m3_rows(a.to(DEV))
         wt = fp8.quantize_weight_e4m3(w.to(torch.bfloat16).t().contiguous().to(DEV))
@@ -364,9 +386,8 @@ def test_gemm_few_row_form_same_bytes(hip_lib, fmt, N, K, resid, out8):
                                      residual=None if r is None else r[s],
                                      silu_cols=None if out8 else (64, 192), **kw)
     full = run(slice(0, M)).view(torch.uint8)
-    for rows in (1, 64, 65, 300):
-        s = slice(200, 200 + rows)
-        assert torch.equal(full[s], run(s).view(torch.uint8)), rows
+    for s in (*(slice(200, 200 + rows) for rows in (1, 64, 65, 300)), slice(M - 50, M)):
+        assert torch.equal(full[s], run(s).view(torch.uint8)), s
 
 
 @pytest.mark.parametrize("N,K,resid", [(256, 128, False), (512, 2048, False), (512, 1536, True), (768, 192, True)])
