@@ -477,7 +477,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_kernel(AttnParams p) {
 
   SeqCtx sc;
   if (!seq_ctx<C::BM>(p, /*heavy_last=*/true, sc)) return;
-  if (sc.tail > 0) zero_tail<D, C::BM>(sc, p.N, p.out, p.o_rs);
+  if (__builtin_expect(sc.tail > 0, 0)) zero_tail<D, C::BM>(sc, p.N, p.out, p.o_rs);
   const int L = sc.L, h = sc.h;
   if constexpr (GENERIC) prefix_block_first<C::BM>(p, sc);
   const int m0 = sc.blk * C::BM;
@@ -853,7 +853,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_fwd_pv8_kernel(AttnParams p)
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   SeqCtx sc;
   if (!seq_ctx(p, /*heavy_last=*/true, sc)) return;
-  if (sc.tail > 0) zero_tail<128>(sc, p.N, p.out, p.o_rs);
+  if (__builtin_expect(sc.tail > 0, 0)) zero_tail<128>(sc, p.N, p.out, p.o_rs);
   const int L = sc.L, h = sc.h;
   const int m0 = sc.blk * C::BM;
   if (m0 >= L) return;
@@ -1419,7 +1419,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
 
   SeqCtx sc;
   if (!seq_ctx(p, /*heavy_last=*/true, sc)) return;
-  if (sc.tail > 0) zero_tail<D>(sc, p.N, p.dq, p.dq_rs);
+  if (__builtin_expect(sc.tail > 0, 0)) zero_tail<D>(sc, p.N, p.dq, p.dq_rs);
   const int L = sc.L, h = sc.h;
   if constexpr (GENERIC) prefix_block_first<C::BM>(p, sc);
   const int m0 = sc.blk * C::BM;
@@ -1481,8 +1481,8 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_kernel(AttnParams p) 
   const int ntiles = (n_end + C::BN - 1) / C::BN;
   int qid[2] = {0, 0};
   if constexpr (GENERIC) {
-    qid[0] = mask_id(mw0 + li, mc);
-    qid[1] = mask_id(mw0 + 16 + li, mc);
+    qid[0] = mask_row_id(mw0 + li, mc);
+    qid[1] = mask_row_id(mw0 + 16 + li, mc);
   }
 
   RowStage<C::BN, D, FP8> k_st, v_st;
@@ -1690,7 +1690,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dq_ws_kernel(AttnParams 
 
   SeqCtx sc;
   if (!seq_ctx(p, /*heavy_last=*/true, sc)) return;
-  if (sc.tail > 0) zero_tail<D>(sc, p.N, p.dq, p.dq_rs);
+  if (__builtin_expect(sc.tail > 0, 0)) zero_tail<D>(sc, p.N, p.dq, p.dq_rs);
   const int L = sc.L, h = sc.h;
   const int m0 = sc.blk * C::BM;
   if (m0 >= L) return;
@@ -1961,7 +1961,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
 
   SeqCtx sc;
   if (!seq_ctx(p, /*heavy_last=*/false, sc)) return;
-  if (sc.tail > 0) {
+  if (__builtin_expect(sc.tail > 0, 0)) {
     zero_tail<D>(sc, p.N, p.dk, p.dk_rs);
     zero_tail<D>(sc, p.N, p.dv, p.dv_rs);
   }
@@ -2193,7 +2193,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_dkdv_kernel(AttnParams p
             if constexpr (MASKED) {
               const int i = m0 + qs * 16 + 4 * g + r, j = kw0 + kt * 16 + li;
               const bool ok = !GENERIC            ? j <= i
-                              : MASKED == MaskGen() ? mask_pair(i, j, mask_id(i, mc), mask_id(j, mc), mc)
+                              : MASKED == MaskGen() ? mask_pair(i, j, mask_row_id(i, mc), mask_id(j, mc), mc)
                                                     : mask_band(i, j, mc);
               pval = ok ? pval : 0.f;
               dval = ok ? dval : 0.f;
@@ -2414,7 +2414,7 @@ __global__ void __launch_bounds__(F8Bwd::NT, 3) hstu_bwd_f8_dkdv_kernel(AttnPara
   SeqCtx sc;
   int half = 0;
   if (!seq_ctx(p, /*heavy_last=*/false, sc, &half)) return;
-  if (sc.tail > 0) {
+  if (__builtin_expect(sc.tail > 0, 0)) {
     if (half == 0) zero_tail<128>(sc, p.N, p.dk, p.dk_rs);
     else zero_tail<128>(sc, p.N, p.dv, p.dv_rs);
   }
@@ -2673,7 +2673,7 @@ __global__ void __launch_bounds__(kThreads, 2) hstu_bwd_f8_dq_kernel(AttnParams 
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   SeqCtx sc;
   if (!seq_ctx(p, /*heavy_last=*/true, sc)) return;
-  if (sc.tail > 0) zero_tail<128>(sc, p.N, p.dq, p.dq_rs);
+  if (__builtin_expect(sc.tail > 0, 0)) zero_tail<128>(sc, p.N, p.dq, p.dq_rs);
   const int L = sc.L, h = sc.h;
   const int qt = sc.blk;
   const int m0 = qt * C::BM;
