@@ -226,7 +226,7 @@ int hstu_attn_bwd_fp8(const void* dout8, const void* dout_e8, int64_t dout_row_s
 /*
  * Its two halves, same arguments, run in order on one stream with one
  * workspace: _dkdv writes dk, dv and leaves the e4m3 dS tiles (and the block
- * schedule, tile prefixes, pre-clamped bias rows and scale maxima) in the
+ * schedule, dQ-block prefix, pre-clamped bias rows and scale maxima) in the
  * workspace; _dq reads them and writes dq and dbias.
  */
 int hstu_attn_bwd_fp8_dkdv(const void* dout8, const void* dout_e8, int64_t dout_row_stride,
@@ -324,7 +324,8 @@ int hstu_fp8_gemm(int a_dtype, const void* A, int64_t lda, const void* W, int64_
                   int silu_begin, int silu_end, hipStream_t stream);
 
 /*
- * bf16 projection GEMM on the same tile kernel: C[m][n] = epilogue(sum_k
+ * bf16 projection GEMM (the few-row, tile and two-workgroup forms of
+ * hstu_fp8_gemm on bf16 rows, by size): C[m][n] = epilogue(sum_k
  * A[m][k] W[n][k]), A [M, K] and W [N, K] row-major bf16 (lda, ldw, ldc, ldr
  * in elements), fp32 accumulate, epilogue as hstu_fp8_gemm without scales
  * (+ bias[n], SiLU on [silu_begin, silu_end), + residual), bf16 C.

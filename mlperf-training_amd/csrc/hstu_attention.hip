@@ -3122,7 +3122,11 @@ __device__ void schedule_block(const int64_t* seq_offsets, int B, int H, int N, 
 // schedule / direct; bf16 forward, backward; H = 4): 8 sequences of up to 1024
 // (256 blocks) 34.8 / 29.2, 78.1 / 69.4; 32 (1024) 38.6 / 35.6, 91.8 / 90.6;
 // 100 of up to 300 (1200) 28.1 / 24.4, 56.9 / 50.0; 64 of up to 1024 (2048)
-// 59.1 / 61.0, 157.7 / 165.8; 128 (4096) 119.5 / 136.2, 317 / 368.
+// 59.1 / 61.0, 157.7 / 165.8; 128 (4096) 119.5 / 136.2, 317 / 368.  e4m3
+// forward, with bf16 P and with FP8 P.V: 8 of 128 .. 1024 33.2 / 27.7, 27.5 / 22.4;
+// 32 of 128 .. 1024 (1024) 40.4 / 41.3, 36.9 / 36.0; 40 of 1024 (1280) 91.3 / 70.5,
+// 78.4 / 60.4; 100 of up to 300 (1200) 28.0 / 22.7, 28.0 / 21.9; 10 of 4096 (1280)
+// 229 / 191, 186 / 157.
 // A call whose set-up launch stays for other work (`prep`: a bias in the
 // backward, the full-FP8 backward's scale maxima) takes it only where the
 // schedule's whole items would leave XCDs idle or uneven: fewer than 16 items.
@@ -3800,7 +3804,7 @@ extern "C" int hstu_attn_bwd_dq(HSTU_BWD_PARAMS) { return attn_bwd_impl(kBwdDq, 
 // ---------------------------------------------------------------------------
 namespace {
 // Workspace: [block schedule][pre-clamped bias rows][partial bias gradients]
-// [scale maxima][dS tile prefix][e4m3 dS tiles].  The tiles are sized by a
+// [scale maxima][e4m3 dS tiles].  The tiles are sized by a
 // bound that needs no lengths: sum_b nq_b (nq_b + 1) / 2 <= (nq_max + 1) / 2 *
 // (ceil(T / 128) + B), nq_max = ceil(N / 128).
 struct F8Ws {

@@ -991,10 +991,11 @@ __global__ void __launch_bounds__(kDuoThreads, 2) fp8_gemm_duo_kernel(GemmParams
 // ring, item protocol and two workgroups per CU as above, on rows of bf16 (a
 // k-step of 128 bytes is 64 elements).
 //
-// What bounds it: the matrix cores (per k-step and wave 1 M MAC against 24 KiB
-// of LDS reads, 0.4 of the LDS rate), so the MFMA is v_mfma_f32_32x32x16_bf16,
-// whose measured rate is 1.62 PFLOP/s against 1.23 for 16x16x32 (whole chip,
-// register operands).  Wave w owns all 128 rows and columns [64 w, 64 w + 64)
+// What bounds it: the matrix cores at long K (busy 61 % of the time at K = 2048;
+// per k-step and wave 1 M MAC against 24 KiB of LDS reads, 0.3 of the LDS rate),
+// at K = 512 (40 %) the output and its epilogue beside them.  So the MFMA is
+// v_mfma_f32_32x32x16_bf16, whose measured rate is 1.62 PFLOP/s against 1.23 for
+// 16x16x32 (whole chip, register operands).  Wave w owns all 128 rows and columns [64 w, 64 w + 64)
 // as 4 x 2 accumulators of 32 x 32 (128 registers); a lane reads chunk
 // 2 kk + lane / 32 of row lane % 32 for the step's MFMA kk, which is conflict
 // free under the same swizzle (16 lanes read 16 consecutive rows).  The W rows
@@ -1005,7 +1006,7 @@ __global__ void __launch_bounds__(kDuoThreads, 2) fp8_gemm_duo_kernel(GemmParams
 // residual 389 -> 300, K = 2048, N = 512 421 -> 326 us (1.04 PFLOP/s); 37 429
 // rows 124 -> 102, 80 -> 70, 96 -> 83 us.  With few rows the tiles no longer
 // cover the chip and a tile's serial k-steps (0.87 us each) are the time; those
-// calls take gemm_few_rows_kernel.
+// calls take gemm_few_rows_kernel, or the tile kernel in between (hstu_bf16_gemm).
 //
 // Column (within a 32-column block) of accumulator element e (0..15) of lane
 // half h; the MFMA's row index is i = 8 (e / 4) + 4 h + e % 4.
@@ -1806,7 +1807,10 @@ hipError_t set_gemm_lds(const void* fn) {
 // (64 wide tiles) 21.6 / 29.0, [8 000, 2048] (126) 39.6 / 30.0; e4m3
 // [4 000, 1536] x [1536, 512] 11.5 / 16.9, [8 000, 1536] 19.9 / 18.2;
 // [1 027, 512] x [512, 2048] (72) bf16 8.2 / 11.5, e4m3 5.8 / 8.6, [4 000, 512]
-// (256) 22.8 / 15.4, 12.0 / 10.7.
+// (256) 22.8 / 15.4, 12.0 / 10.7.  Against the producer/consumer form, which e4m3
+// takes above the line at N <= 512 without a residual: [4 000, 512] x [512, 512]
+// (64) 5.4 / 8.9, [5 120, 512] (80) 7.1 / 9.1, [5 120, 2048] 16.9 / 17.6.  bf16 draws
+// a further line (hstu_bf16_gemm).
 constexpr int kFewMaxWideTiles = 80;
 bool few_rows(int M, int N) { return (int64_t)((M + kBM - 1) / kBM) * (N / kWideBN) <= kFewMaxWideTiles; }
 // 128 x 128 tiles that the tile kernel runs in one round, one a CU.
@@ -1932,7 +1936,7 @@ extern "C" int hstu_fp8_gemm(int a_dtype, const void* A, int64_t lda, const void
 extern "C" int hstu_bf16_gemm(const void* A, int64_t lda, const void* W, int64_t ldw, const void* bias,
                               const void* residual, int64_t ldr, void* C, int64_t ldc, int M, int N, int K,
                               int silu_begin, int silu_end, hipStream_t stream) {
-  // the tile kernel on bf16 rows: k counted in bytes (128-byte k-steps)
+  // bf16 rows: k counted in bytes (128-byte k-steps)
   if (M < 0 || N <= 0 || K <= 0 || N % kBN != 0 || (2 * K) % kBK != 0 || !A || !W || !C) return HSTU_E_BAD_ARG;
   if (lda < K || ldw < K || ldc < N || (residual && ldr < N)) return HSTU_E_BAD_ARG;
   if (lda % 8 != 0 || ldw % 8 != 0 || ldc % 4 != 0 || (residual && ldr % 4 != 0) ||

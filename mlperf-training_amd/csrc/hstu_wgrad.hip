@@ -19,8 +19,8 @@
 // k(token)-contiguous fragments with the same token order in both operands.
 // The MFMA (v_mfma_f32_16x16x32_bf16, 16x16x128_f8f6f4) runs with B as its A
 // operand, so a lane's result is 4 consecutive n2 of one n1 row.
-// What bounds it: the matrix cores and, close behind, the transposed reads (for
-// fp8 1 900 LDS cycles against 2 050 MFMA cycles a step), so the two must
+// What bounds it: the transposed reads and the MFMAs, close to equal (for fp8
+// 1 900 LDS cycles against 2 050 MFMA cycles a step), so the two must
 // overlap although the eight waves meet at a barrier every step: the
 // fragments roll.  A fragment's registers are refilled with the next step's as
 // soon as its last MFMA is issued, so the LDS reads of step k + 1 run under the
@@ -31,11 +31,14 @@
 // the transposed reads over all banks.
 // Measured, product + second pass, against operands loaded through registers and
 // read from padded LDS all at once behind the barrier, in us:
-//                        512 x 2048        1536 x 512
-//   bf16 T = 162 251   361.5 -> 346.0    254.1 -> 231.7  (983 / 1 101 TFLOP/s)
-//   bf16 T =  37 429    99.9 ->  91.5     73.7 ->  67.7
-//   fp8  T = 162 251   176.5 -> 175.0    133.5 -> 135.0  (no gain: one code for
-//   fp8  T =  37 429    57.6 ->  57.5     47.5 ->  47.7   both formats)
+//                                       512 x 2048      1536 x 512
+//   bf16 T = 162 251                   327 -> 296      256 -> 232  (1.15 / 1.10 PFLOP/s)
+//   bf16 T = 162 251, column sums too  346 -> 327      265 -> 249
+//   bf16 T =  37 429                  95.2 -> 87.7    76.8 -> 70.9
+//   fp8  T = 162 251                   183 -> 176      140 -> 137
+//   fp8  T =  37 429                  57.9 -> 55.5    48.9 -> 47.4
+// Matrix cores busy 61 % (bf16) and 46 % (fp8) of the time, the LDS at 0.55 and
+// 0.43 of its read rate: the two overlap, but not wholly across the barrier.
 // Workgroups are numbered so that the tiles of one token range run on one XCD
 // and share its L2.  With split > 1 every workgroup writes an fp32 partial
 // tile; a second kernel sums the splits in a fixed order, applies sa * sb and

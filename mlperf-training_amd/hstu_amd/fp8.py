@@ -251,8 +251,8 @@ def fp8_gemm(a8: torch.Tensor, a_scale: torch.Tensor, weight: Weight, *, bias: O
 def bf16_gemm(a: torch.Tensor, w_nk: torch.Tensor, *, bias: Optional[torch.Tensor] = None,
               residual: Optional[torch.Tensor] = None, silu_cols: Optional[Tuple[int, int]] = None,
               out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """bf16 C = epilogue(a @ w_nk^T) on the HIP tile kernel (``hstu_bf16_gemm``):
-    a [M, K], w_nk [N, K] (the weight with the contraction index contiguous),
+    """bf16 C = epilogue(a @ w_nk^T) on the HIP GEMM (``hstu_bf16_gemm``, few-row,
+    tile or two-workgroup form by size; the same bytes in each): a [M, K], w_nk [N, K] (the weight with the contraction index contiguous),
     optional bf16 bias [N], residual [M, N], SiLU on a column range.  ``out``:
     an [M, N] bf16 destination with unit column stride (e.g. columns of a
     wider buffer)."""
