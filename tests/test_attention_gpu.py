@@ -720,8 +720,7 @@ def _cut(x, lengths, N):
 
 def test_full_fp8_backward_rows_past_max_seq_len(hip_lib):
     """A sequence longer than max_seq_len: the full-FP8 backward leaves its
-    dq, dk and dv rows past N zero (the set-up launch zeroes them; the
-    gradient buffers start as NaN) and the other rows equal, bitwise, the
+    dq, dk and dv rows past N zero (the gradient buffers start as NaN) and the other rows equal, bitwise, the
     same call on the batch with that sequence cut at N."""
     ops = _ops()
     H, D = 2, 128
@@ -811,15 +810,18 @@ def test_direct_grid_same_bytes_past_the_bias_range(hip_lib, far, D, win, ctx):
                                          ("e4m3", 128, 2), ("full", 128, 0)])
 @pytest.mark.parametrize("pad", [0, 4])
 @pytest.mark.parametrize("N", [64, 300])
-def test_direct_grid_long_tails(hip_lib, kind, D, mask, pad, N):
+@pytest.mark.parametrize("empty", [0, 1300])
+def test_long_tails(hip_lib, kind, D, mask, pad, N, empty):
     """Rows past max_seq_len N, many times N of them, on a direct grid (each of
-    an item's blocks zeroes its share): zero in out, dq, dk and dv, and nothing
-    beside them; gradients as views of wider buffers, 16-byte aligned or not."""
+    an item's blocks zeroes its share) and on the scheduled one (the set-up
+    launch does): zero in out, dq, dk and dv, and nothing beside them; gradients
+    as views of wider buffers, 16-byte aligned or not."""
     ops = _ops()
     H, lengths = 2, [N + 1, 3, N, 5 * N + 77, 0, 2 * N + 130]
     q, k, v, offs = _case(lengths, H, D, seed=N)
     T = q.shape[0]
     q, k, v, dout = (t.to(DEV) for t in (q, k, v, q.flip(0)))
+    offs = orc.offsets_from_lengths(lengths + [0] * empty)
     scales = [None] * 3
     if kind != "bf16":
         q, k, v = ((t.float() * 100).to(torch.float8_e4m3fn) for t in (q, k, v))
